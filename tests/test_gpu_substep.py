@@ -175,6 +175,17 @@ def test_failed_substep_leaves_the_scene(ctx):
     assert 0 < rep["max_speed"] < 10.0
 
 
+@pytest.mark.parametrize("n", [1, 63, 255, 256, 257, 1000])
+def test_download_returns_the_upload(ctx, n):
+    rng = np.random.default_rng(n)
+    x, v, c = rng.random((n, 3)), rng.normal(size=(n, 3)), rng.normal(size=(n, 9))
+    assert ctx.scene_upload(O.geometry((0.0, 0.0, 0.0), 0.1), x, v, c, 1.0) == H.OK
+    s, gx, gv, gc, gj, gf = ctx.substep_download(n)
+    assert s == H.OK
+    assert np.array_equal(gx, x) and np.array_equal(gv, v) and np.array_equal(gc, c)
+    assert np.all(gj == 1.0) and np.all(gf == 0)
+
+
 def floor_record():
     return SC.obstacle_record(O.halfspace((0.0, 1.0, 0.0), 0.0), R.OBSTACLE)
 
