@@ -668,7 +668,7 @@ int fl_reserve(fl_ctx* ctx) {
     FL_TRY(grow(&B.cells, &B.cap[10], nc));
     FL_TRY(grow(&B.faces, &B.cap[11], 6 * nc));
     FL_TRY(grow(&B.needs, &B.cap[12], nc));
-    FL_TRY(grow(&B.counts, &B.cap[13], 4));
+    FL_TRY(grow(&B.counts, &B.cap[13], 5));
     FL_TRY(grow(&B.phi, &B.cap[14], 9 * nc));
     FL_TRY(grow(&B.work, &B.cap[15], nc));
     FL_TRY(grow(&B.uncut, &B.cap[16], 2));
@@ -1162,7 +1162,7 @@ int fl_freeze_geometry(fl_ctx* ctx, const fl_freeze_inputs* inputs, fl_frozen_ce
   FL_TRY(grow(&B.cells, &B.cap[10], nc_in));
   FL_TRY(grow(&B.faces, &B.cap[11], 6 * nc_in));
   FL_TRY(grow(&B.needs, &B.cap[12], nc_in));
-  FL_TRY(grow(&B.counts, &B.cap[13], 4));
+  FL_TRY(grow(&B.counts, &B.cap[13], 5));
   FL_TRY(grow(&B.phi, &B.cap[14], 9 * nc_in));
   FL_TRY(grow(&B.work, &B.cap[15], nc_in));
   FL_TRY(grow(&B.uncut, &B.cap[16], 2));

@@ -303,7 +303,7 @@ struct FreezeDevice {
   fl_frozen_cell* cells;  // ncand
   fl_frozen_face* faces;  // 6 * ncand
   uint8_t* needs;         // ncand
-  uint64_t* counts;       // 4: kept cells, unique faces, curvature needed, listed cut cells
+  uint64_t* counts;       // 5: kept cells, unique faces, curvature needed, cells listed from the front / back of work
   double* phi;            // 9 * ncand: corner and centre samples of the cut cells
   uint64_t* work;         // ncand: the cut cells
   double* uncut_volume;   // 2: the uncut cell's volume, plane mode then sampled mode

@@ -368,7 +368,7 @@ int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep) {
   FL_TRY(grow_to(&B.cells, &B.cap[10], ncand));
   FL_TRY(grow_to(&B.faces, &B.cap[11], 6 * ncand));
   FL_TRY(grow_to(&B.needs, &B.cap[12], ncand));
-  FL_TRY(grow_to(&B.counts, &B.cap[13], 4));
+  FL_TRY(grow_to(&B.counts, &B.cap[13], 5));
   FL_TRY(grow_to(&B.phi, &B.cap[14], 9 * ncand));
   FL_TRY(grow_to(&B.work, &B.cap[15], ncand));
   FL_TRY(grow_to(&B.uncut, &B.cap[16], 2));

@@ -164,6 +164,24 @@ def test_sphere(ctx, case):
     print("freeze", case, len(p.candidates), "candidates", ctx.last.kernel_ms, "ms", flush=True)
 
 
+@pytest.mark.parametrize("eps", [0.0, 1e-17, 1e-12, 1e-10, 1e-7])
+@pytest.mark.parametrize("slab", [False, True])
+def test_planes_beside_the_lattice(ctx, slab, eps):
+    """Planes on and just beside a lattice plane: cells that a plane clearly misses are clipped by the liquid
+    surface alone, the ones it may touch by both, with the same bits; 1 to 12 candidates fill whole and
+    part groups of lanes."""
+    for side in (-1.0, 1.0):
+        c = 9.0 / 20 + side * eps
+        obstacle = O.slab((1.0, 0.0, 0.0), c, 0.01, (0.5, 0.0, 0.0)) if slab else O.halfspace((1.0, 0.0, 0.0), c)
+        check(ctx, sphere(n=20, obstacle=obstacle))
+    if not slab and eps == 0.0:
+        p = sphere(n=20)
+        whole = p.candidates
+        for count in (1, 9, 10, 11, 12):
+            p.candidates = whole[:count]
+            assert check(ctx, p) in (O.OK, O.FAILED_PRECONDITION)
+
+
 def test_freeze_then_links(ctx):
     """The device's frozen view, with the problem's centre samples, gives the oracle's links of the
     oracle's freeze."""

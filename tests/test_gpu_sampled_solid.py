@@ -125,6 +125,15 @@ def test_config5_solids(ctx, mode):
         assert faces["has_prescribed_wall_flux"].all()
 
 
+@pytest.mark.parametrize("rule", [2, 3])
+@pytest.mark.parametrize("mode", ["corners", "halfspace"])
+def test_surface_cells_away_from_solids(ctx, mode, rule):
+    """Split rules 2 and 3 clip cells clear of every solid by the liquid surface alone: the same bits."""
+    p = config5_problem(n=30, mode=mode)
+    p.split_rule = rule
+    check(ctx, p)
+
+
 def test_sampled_plane_matches_halfspace(ctx):
     normal, plane = (0.6, 0.8, 0.0), 0.1
     liquid = lambda x, y, z: 0.37 * x + 0.21 * y - 0.13 * z - 0.9
