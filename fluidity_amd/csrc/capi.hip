@@ -517,19 +517,6 @@ int stage_particles(fl_ctx* ctx, const fl_particle* particles, size_t n, bool de
 
 }  // namespace
 
-namespace fl {
-int viscosity_reserve(fl_ctx* ctx, uint64_t n, uint64_t nr, uint64_t nf, ViscosityDevice* out) {
-  FL_TRY(grow_viscosity(ctx, std::max<uint64_t>(n, 1), std::max<uint64_t>(nr, 1), std::max<uint64_t>(nf, 1)));
-  *out = viscosity_device(ctx);
-  return FL_OK;
-}
-int viscosity_reserve_terms(fl_ctx* ctx, uint64_t nt, ViscosityDevice* out) {
-  FL_TRY(grow_viscosity_terms(ctx, nt));
-  *out = viscosity_device(ctx);
-  return FL_OK;
-}
-}  // namespace fl
-
 extern "C" {
 
 int fl_create(const fl_capacities* capacities, int device, fl_ctx** out) {
@@ -579,6 +566,7 @@ void fl_destroy(fl_ctx* ctx) {
   fl::release_field(ctx);
   fl::release_substep(ctx);
   fl::release_coupled(ctx);
+  fl::release_uniform(ctx);
   release(ctx);
   for (hipEvent_t e : ctx->stage)
     if (e) (void)hipEventDestroy(e);

@@ -171,6 +171,7 @@ struct fl_ctx {
   void* field = nullptr;      // FieldBuffers (field.hip)
   void* substep = nullptr;    // SubstepBuffers (substep.hip)
   void* coupled = nullptr;    // CoupledBuffers (coupled.hip)
+  void* uniform = nullptr;    // UniformBuffers (uniform.hip)
 };
 
 namespace fl {
@@ -389,10 +390,26 @@ int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& v,
                   const fl_pressure_options& options, bool jacobi, CoupledResult* out);
 int coupled_outputs(fl_ctx* ctx, const double** p, const double** u, const double** defects);
 void release_coupled(fl_ctx* ctx);
-// The context's viscosity arrays (capi.hip) sized for n cells, nr rows and nf faces, then for nt packed
-// terms; *out views them.
-int viscosity_reserve(fl_ctx* ctx, uint64_t n, uint64_t nr, uint64_t nf, ViscosityDevice* out);
-int viscosity_reserve_terms(fl_ctx* ctx, uint64_t nt, ViscosityDevice* out);
+// The velocity block of one dynamic viscosity on the full-cell strain rows of the pressure cells, without
+// rows (uniform.hip): face vectors in owned-slot order on the context's grid.
+struct UniformBlock {
+  double *inertia, *rhs, *v, *diag;
+};
+// Sizes and clears the block's arrays for the context's blocks; then, with the inertia of the links set,
+// the rows' structure, the Jacobi diagonal and the prescribed strains in base (link order); *rows counts the
+// strain rows that AssembleFullCellMacStrain3D would form. Failures also go to err (two words).
+int uniform_prepare(fl_ctx* ctx, UniformBlock* out);
+int uniform_rows(fl_ctx* ctx, const CoupledSystem& S, const fl_pressure_cell* cells, double mu, double h, double dt,
+                 double* base, uint64_t* err, uint64_t* rows);
+// As pcg_viscous_block, for the right-hand side in the block's rhs.
+int uniform_solve(fl_ctx* ctx, double max_rhs, uint64_t max_iterations, double relative_tolerance,
+                  uint64_t* iterations, double* max_residual);
+void release_uniform(fl_ctx* ctx);
+// coupled_rows and coupled_solve on that block.
+int coupled_uniform_rows(fl_ctx* ctx, const CoupledSystem& S, const fl_pressure_cell* cells, double mu, double h,
+                         double dt, UniformBlock* block, uint64_t* rows);
+int coupled_uniform_solve(fl_ctx* ctx, const CoupledSystem& S, const UniformBlock& U, double dt,
+                          const fl_pressure_options& options, bool jacobi, CoupledResult* out);
 
 // The device substep (substep.hip).
 int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep);

@@ -173,9 +173,12 @@ __global__ void k_remap(fl_strain_row* rows, uint64_t nr, const uint64_t* slot, 
   }
 }
 
+// Place of link f in the velocity block's face vectors: the link order, or its owned slot (uniform.hip).
+__device__ inline uint64_t place(const uint64_t* at, uint64_t f) { return at ? at[f] : f; }
+
 // Face inertia and the base momentum M u* + dt A lift (:185-205); lift is the internal jump, or the
 // exterior pressure signed by the missing endpoint.
-__global__ void k_setup(uint64_t nf, double dt, const double* area, const double* scale, const double* ustar,
+__global__ void k_setup(uint64_t nf, const uint64_t* at, double dt, const double* area, const double* scale, const double* ustar,
                         const double* lift, const int32_t* kind, const int32_t* tail, double* inertia, double* base,
                         uint64_t* err) {
   const uint64_t f = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
@@ -190,7 +193,7 @@ __global__ void k_setup(uint64_t nf, double dt, const double* area, const double
     else if (kind[f] == 2) l = tail[f] >= 0 ? -lift[f] : lift[f];
     b = m * ustar[f] + step_area * l;
   }
-  inertia[f] = m;
+  inertia[place(at, f)] = m;
   base[f] = b;
 }
 
@@ -215,13 +218,14 @@ __global__ void k_eliminate(const fl_strain_row* rows, uint64_t nr, const double
 
 // Effective conductance k M / (M + dt sum w c^2) of each open face (:213-224); the base momentum must
 // be finite.
-__global__ void k_effective(uint64_t nf, const double* conductance, const double* inertia, const double* vdiag,
+__global__ void k_effective(uint64_t nf, const uint64_t* at, const double* conductance, const double* inertia, const double* vdiag,
                             const double* base, double* eff, uint64_t* err) {
   const uint64_t f = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
   if (f >= nf) return;
+  const uint64_t i = place(at, f);
   double e = 0.0;
-  if (inertia[f] != 0.0) {
-    e = conductance[f] * (inertia[f] / vdiag[f]);
+  if (inertia[i] != 0.0) {
+    e = conductance[f] * (inertia[i] / vdiag[i]);
     if (!(isfinite(e) && e > 0.0)) report(err, f, FL_OUT_OF_RANGE);
   }
   if (!isfinite(base[f])) report(err, f, FL_OUT_OF_RANGE);
@@ -239,7 +243,7 @@ __global__ void k_pressure_diagonal(uint64_t nc, const int32_t* cell_faces, cons
 
 // Velocity block right-hand side for pressure p: base (physical only) + dt A (p_tail - p_head), missing
 // endpoints at zero (:281-297); partial maxima of |rhs| in slot 2.
-__global__ void k_momentum(uint64_t nf, double dt, const double* base, const double* area, const int32_t* tail,
+__global__ void k_momentum(uint64_t nf, const uint64_t* at, double dt, const double* base, const double* area, const int32_t* tail,
                            const int32_t* head, const double* p, int physical, double* rhs, double* partial) {
   double v[4] = {0.0, 0.0, 0.0, 0.0};
   for (uint64_t f = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; f < nf; f += uint64_t(gridDim.x) * blockDim.x) {
@@ -249,7 +253,7 @@ __global__ void k_momentum(uint64_t nf, double dt, const double* base, const dou
       const double ph = head[f] >= 0 ? p[head[f]] : 0.0;
       m += dt * area[f] * (pt - ph);
     }
-    rhs[f] = m;
+    rhs[place(at, f)] = m;
     v[2] = fmax(v[2], fabs(m));
   }
   group_reduce4(v, partial);
@@ -268,7 +272,7 @@ struct Neumaier {
 // AccumulateConstraint (:83-134) per cell: -target (physical), compliance (p - p_prev or p), and the
 // outward open flux A u of the six incident links plus their wall flux (physical). Non-physical calls
 // zero the gauge cells (the responses). Partials: slot 0 sum r^2, slot 3 max |r| / V.
-__global__ void k_constraint(uint64_t nc, const int32_t* cell_faces, const int32_t* tail, const double* area,
+__global__ void k_constraint(uint64_t nc, const uint64_t* at, const int32_t* cell_faces, const int32_t* tail, const double* area,
                              const double* wall, const double* target, const double* comp, const double* prev,
                              const double* volume, const uint8_t* flag, const double* p, const double* u,
                              int physical, double* out, double* partial, uint64_t* err) {
@@ -281,7 +285,7 @@ __global__ void k_constraint(uint64_t nc, const int32_t* cell_faces, const int32
     for (int j = 0; j < 6; ++j) {
       const int32_t f = cell_faces[6 * c + j];
       const double sign = tail[f] == c ? 1.0 : -1.0;
-      flux.add(sign * (area[f] * u[f]));
+      flux.add(sign * (area[f] * u[place(at, f)]));
       if (physical) flux.add(sign * wall[f]);
     }
     double r = flux.total();
@@ -351,9 +355,12 @@ __global__ void k_step(uint64_t n, const double* scal, double* resp, double* dir
 
 // Accepted velocities: the solved ones on open faces, the wall normal velocity on eliminated ones; the
 // defects r / V.
-__global__ void k_accept(uint64_t nf, const double* inertia, const double* v, const double* uwall, double* u) {
+__global__ void k_accept(uint64_t nf, const uint64_t* at, const double* inertia, const double* v, const double* uwall,
+                         double* u) {
   const uint64_t f = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  if (f < nf) u[f] = inertia[f] == 0.0 ? uwall[f] : v[f];
+  if (f >= nf) return;
+  const uint64_t i = place(at, f);
+  u[f] = inertia[i] == 0.0 ? uwall[f] : v[i];
 }
 __global__ void k_defects(uint64_t nc, const double* res, const double* volume, double* d) {
   const uint64_t c = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
@@ -412,22 +419,46 @@ int coupled_rows(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V, 
   if (nr) k_remap<<<grid_for(nr), kThreads, 0, s>>>(V.rows, nr, S.slot, S.nf, B.err);
   FL_HIP(hipGetLastError());
   FL_TRY(read_err(ctx, B));
-  k_setup<<<grid_for(S.nf), kThreads, 0, s>>>(S.nf, dt, S.area, S.scale, S.ustar, S.lift, S.kind, S.tail,
+  k_setup<<<grid_for(S.nf), kThreads, 0, s>>>(S.nf, nullptr, dt, S.area, S.scale, S.ustar, S.lift, S.kind, S.tail,
                                               const_cast<double*>(V.inertia), B.base, B.err);
   if (nr) k_eliminate<<<grid_for(nr), kThreads, 0, s>>>(V.rows, nr, V.inertia, S.uwall, dt, B.base);
   FL_HIP(hipGetLastError());
   return read_err(ctx, B);
 }
 
-int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V, uint64_t nr, uint64_t nt, double dt,
-                  const fl_pressure_options& o, bool jacobi, CoupledResult* out) {
+int coupled_uniform_rows(fl_ctx* ctx, const CoupledSystem& S, const fl_pressure_cell* cells, double mu, double h,
+                         double dt, UniformBlock* block, uint64_t* rows) {
+  FL_TRY(ensure(ctx, S.nc, S.nf));
+  auto& B = *static_cast<CoupledBuffers*>(ctx->coupled);
+  hipStream_t s = ctx->stream;
+  FL_TRY(uniform_prepare(ctx, block));
+  k_reset<<<1, 64, 0, s>>>(B.err);
+  k_setup<<<grid_for(S.nf), kThreads, 0, s>>>(S.nf, S.slot, dt, S.area, S.scale, S.ustar, S.lift, S.kind, S.tail,
+                                              block->inertia, B.base, B.err);
+  FL_HIP(hipGetLastError());
+  FL_TRY(uniform_rows(ctx, S, cells, mu, h, dt, B.base, B.err, rows));
+  return read_err(ctx, B);
+}
+
+namespace {
+
+// A velocity block by its face vectors (M, rhs, velocity, diagonal of H), their place per link, and its
+// solve to a relative tolerance of the largest right-hand side.
+struct VelocityBlock {
+  const double* inertia;
+  double *rhs, *v;
+  const double* diag;
+  const uint64_t* at;
+};
+
+template <class Solve>
+int gcr_solve(fl_ctx* ctx, const CoupledSystem& S, const VelocityBlock& V, double dt, const fl_pressure_options& o,
+              bool jacobi, CoupledResult* out, Solve solve) {
   auto& B = *static_cast<CoupledBuffers*>(ctx->coupled);
   hipStream_t s = ctx->stream;
   const uint64_t nc = S.nc, nf = S.nf;
-  *out = CoupledResult{};
-  FL_TRY(pack_viscous_block(ctx, V, nr, nf, nt, dt));  // V.diag = M + dt sum w c^2
   k_reset<<<1, 64, 0, s>>>(B.err);
-  k_effective<<<grid_for(nf), kThreads, 0, s>>>(nf, S.conductance, V.inertia, V.diag, B.base, B.eff, B.err);
+  k_effective<<<grid_for(nf), kThreads, 0, s>>>(nf, V.at, S.conductance, V.inertia, V.diag, B.base, B.eff, B.err);
   k_pressure_diagonal<<<grid_for(nc), kThreads, 0, s>>>(nc, S.cell_faces, S.comp, B.eff, B.pdiag);
   if (!jacobi) FL_TRY(coupled_coefficients(ctx, B.eff));
   k_zero<<<grid_for(nc), kThreads, 0, s>>>(nc, B.zero);
@@ -438,8 +469,8 @@ int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V,
 
   // One velocity solve for pressure p; V.v holds the velocities.
   auto solve_velocity = [&](const double* p, bool physical) -> int {
-    k_momentum<<<gf, kThreads, 0, s>>>(nf, dt, B.base, S.area, S.tail, S.head, p, physical ? 1 : 0,
-                                       const_cast<double*>(V.rhs), B.partial);
+    k_momentum<<<gf, kThreads, 0, s>>>(nf, V.at, dt, B.base, S.area, S.tail, S.head, p, physical ? 1 : 0, V.rhs,
+                                       B.partial);
     k_finish4<<<1, kThreads, 0, s>>>(B.partial, gf, B.scal, 0);
     FL_HIP(hipGetLastError());
     FL_HIP(hipMemcpyAsync(B.host, B.scal, 4 * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -451,7 +482,7 @@ int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V,
     // The physical solves to the reference's 1e-10; on the V-cycle path a direction's solve to 1e-5, as
     // GCR keeps the response it measures and acceptance rests on a fresh physical solve.
     const double tolerance = physical || jacobi ? 1e-10 : 1e-5;
-    FL_TRY(pcg_viscous_block(ctx, V, nr, nf, max_rhs, 256, tolerance, &it, &mr));
+    FL_TRY(solve(max_rhs, tolerance, &it, &mr));
     ++out->velocity_solves;
     out->velocity_iterations += it;
     if (physical) out->max_momentum_residual = mr;
@@ -459,7 +490,7 @@ int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V,
   };
   // Constraint of (p, V.v) into dst; returns the residual L2 and max |r| / V (physical) in B.host[0..1].
   auto constraint = [&](const double* p, bool physical, double* dst) -> int {
-    k_constraint<<<gc, kThreads, 0, s>>>(nc, S.cell_faces, S.tail, S.area, S.wall, S.target, S.comp, S.prev,
+    k_constraint<<<gc, kThreads, 0, s>>>(nc, V.at, S.cell_faces, S.tail, S.area, S.wall, S.target, S.comp, S.prev,
                                          S.volume, S.flag, p, V.v, physical ? 1 : 0, dst, B.partial, B.err);
     k_finish4<<<1, kThreads, 0, s>>>(B.partial, gc, B.scal, 4);
     FL_HIP(hipGetLastError());
@@ -533,7 +564,7 @@ int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V,
       continue;
     }
     if (gates) {
-      k_accept<<<grid_for(nf), kThreads, 0, s>>>(nf, V.inertia, V.v, S.uwall, B.u);
+      k_accept<<<grid_for(nf), kThreads, 0, s>>>(nf, V.at, V.inertia, V.v, S.uwall, B.u);
       k_defects<<<grid_for(nc), kThreads, 0, s>>>(nc, B.res, S.volume, B.defects);
       FL_HIP(hipGetLastError());
       FL_HIP(hipStreamSynchronize(s));
@@ -567,6 +598,29 @@ int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V,
   }
   FL_TRY(coupled_error(ctx));
   return FL_ABORTED;
+}
+
+}  // namespace
+
+int coupled_solve(fl_ctx* ctx, const CoupledSystem& S, const ViscosityDevice& V, uint64_t nr, uint64_t nt, double dt,
+                  const fl_pressure_options& o, bool jacobi, CoupledResult* out) {
+  *out = CoupledResult{};
+  FL_TRY(pack_viscous_block(ctx, V, nr, S.nf, nt, dt));  // V.diag = M + dt sum w c^2
+  const VelocityBlock block{V.inertia, const_cast<double*>(V.rhs), V.v, V.diag, nullptr};
+  return gcr_solve(ctx, S, block, dt, o, jacobi, out,
+                   [&](double max_rhs, double tolerance, uint64_t* it, double* mr) {
+                     return pcg_viscous_block(ctx, V, nr, S.nf, max_rhs, 256, tolerance, it, mr);
+                   });
+}
+
+int coupled_uniform_solve(fl_ctx* ctx, const CoupledSystem& S, const UniformBlock& U, double dt,
+                          const fl_pressure_options& o, bool jacobi, CoupledResult* out) {
+  *out = CoupledResult{};
+  const VelocityBlock block{U.inertia, U.rhs, U.v, U.diag, S.slot};
+  return gcr_solve(ctx, S, block, dt, o, jacobi, out,
+                   [&](double max_rhs, double tolerance, uint64_t* it, double* mr) {
+                     return uniform_solve(ctx, max_rhs, 256, tolerance, it, mr);
+                   });
 }
 
 int coupled_outputs(fl_ctx* ctx, const double** p, const double** u, const double** defects) {

@@ -154,16 +154,6 @@ __global__ void k_sample_solid(const fl_center_distance* corners, uint64_t n, do
   out[i] = c;
 }
 
-// MacViscosityCell3D of the pressure cells with one dynamic viscosity.
-__global__ void k_viscosity_cells(const fl_pressure_cell* cells, uint64_t n, double mu, fl_viscosity_cell* out) {
-  const uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  if (i >= n) return;
-  fl_viscosity_cell c{};
-  c.cell_index = cells[i].cell_index;
-  c.dynamic_viscosity = mu;
-  out[i] = c;
-}
-
 // Accepted link velocities into their grid slots.
 __global__ void k_scatter_links(const uint64_t* slot, const double* u, uint64_t nf, double* unew) {
   const uint64_t f = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
@@ -496,19 +486,12 @@ int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep) {
     popt.preconditioner = 0;
     CoupledSystem S{};
     STAGE(6, coupled_prepare_device(ctx, B.pcells, nc, B.pfaces, nf, dt, popt, &S));
-    ViscosityDevice V{};
-    STAGE(6, viscosity_reserve(ctx, nc, 6 * nc, nf, &V));
-    k_viscosity_cells<<<grid_for(nc), kThreads, 0, s>>>(B.pcells, nc, o.dynamic_viscosity,
-                                                        const_cast<fl_viscosity_cell*>(V.cells));
-    FL_HIP(hipGetLastError());
-    uint64_t nr = 0, nt = 0;
-    STAGE(6, assemble_strain(ctx, V, nc, h, &nr));
-    rep.strain_rows = nr;
-    STAGE(6, coupled_rows(ctx, S, V, nr, dt));
-    STAGE(6, weight_viscous_rows(ctx, V, nr, nf, dt, &nt));
-    STAGE(6, viscosity_reserve_terms(ctx, nt, &V));
+    UniformBlock U{};
+    uint64_t rows = 0;
+    STAGE(6, coupled_uniform_rows(ctx, S, B.pcells, o.dynamic_viscosity, h, dt, &U, &rows));
+    rep.strain_rows = rows;
     CoupledResult cr{};
-    const int cst = coupled_solve(ctx, S, V, nr, nt, dt, popt, jacobi, &cr);
+    const int cst = coupled_uniform_solve(ctx, S, U, dt, popt, jacobi, &cr);
     rep.viscous.pressure_iterations = cr.iterations;
     rep.viscous.constraint_residual_l2 = cr.residual_l2;
     rep.viscous.initial_constraint_residual_l2 = cr.initial_residual_l2;

@@ -249,3 +249,31 @@ def test_substep_chain_with_solids_and_viscosity(ctx, jacobi):
             assert dx <= 1e-9 * h and dv <= 1e-7 * speed and dj <= 1e-10
         else:
             assert dx <= 1e-6 * h and dv <= 1e-4 * speed and dj <= 1e-7
+
+
+@pytest.mark.parametrize("n", [13, 18, 21])
+def test_uniform_viscosity_on_odd_grids(ctx, n):
+    """One stirred viscous substep on grids whose blocks the domain cuts, with the reference's Jacobi
+    preconditioner: the row-free velocity block follows the oracle's assembled rows (counts, iterations)."""
+    sc, solid = scenes.stirred_dam_break(n, seed=n, paddle_half_extent=(0.15, 0.1, 0.06), paddle_pivot=(0.35, 0.12, 0.5))
+    geom = O.geometry((0.0, 0.0, 0.0), sc.h)
+    h, radius, dt = sc.h, 0.9 * sc.h, 0.25 * sc.h
+    floor = O.halfspace((0.0, 1.0, 0.0), -0.25 * h)
+    assert ctx.scene_upload(geom, sc.positions, sc.velocities, sc.slopes.reshape(-1, 9), sc.mass) == H.OK
+    popt = H.pressure_options(levels=2, sweeps=2)
+    popt["preconditioner"] = 2
+    o = H.substep_options(dt, field_radius=radius, capacity=1 << 16, obstacle=SC.obstacle_record(floor, R.OBSTACLE),
+                          pressure=popt, dynamic_viscosity=1.0)
+    o["solid"] = solid_record(solid, 0.0)
+    o["solid"]["split_rule"] = 3
+    s, rep = ctx.substep(o)
+    assert s == H.OK, (s, int(rep["stage"]))
+    st = SC.State(sc.positions, sc.velocities, sc.slopes, sc.mass)
+    st, info = SC.oracle_substep(geom, st, dt, radius, floor, None, capacity=1 << 16, solid=solid, viscosity=1.0,
+                                 split_rule=3)
+    assert rep["frozen_cells"] == len(info["frozen_cells"]) and rep["strain_rows"] == len(info["rows"])
+    want_it = int(info["projection"]["diagnostics"]["pressure_iterations"])
+    assert abs(int(rep["viscous"]["pressure_iterations"]) - want_it) <= 1
+    s, x, vel, c, j, f = ctx.substep_download(len(st.x))
+    speed = max(float(np.abs(st.v).max()), 1e-3)
+    assert s == H.OK and np.abs(x - st.x).max() <= 1e-9 * h and np.abs(vel - st.v).max() <= 1e-7 * speed
