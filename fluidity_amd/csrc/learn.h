@@ -47,13 +47,15 @@ struct LearnState {
   float* data_target = nullptr;    // [data_cap][512]
   uint64_t data_cap = 0, ndata = 0;
   int collect_every = 0;  // > 0: the MGPCG solver appends (residual, correction) pairs every k-th iteration
+  float* packed = nullptr;   // [2 * net_param_count()] weights packed for the FP32 convolutions
   uint8_t* frags = nullptr;  // [net_fragment_bytes()] BF16 weights in matrix-core operand order
 };
 
 uint64_t net_param_count();
 // FP32 forward pass over nt tiles whose inputs are at kActIn of each record (training, and the FP32
-// reference of the inference path); every activation is kept in the records for the backward pass.
-int net_forward(hipStream_t s, const float* params, float* act, uint64_t nt);
+// reference of the inference path); every activation is kept in the records for the backward pass. The
+// weights are packed into packed (2 * net_param_count() floats) on every call.
+int net_forward(hipStream_t s, const float* params, float* packed, float* act, uint64_t nt);
 // BF16 inference over nt tiles: reads the inputs at kActIn and writes the output at kActOut of each
 // record, with the whole network of a tile in one workgroup on the matrix cores. frags holds
 // net_fragment_bytes() bytes of device memory; the weights are repacked into it on every call.
@@ -62,9 +64,10 @@ int net_infer(hipStream_t s, const float* params, void* frags, float* act, uint6
 // Masked loss: scalars[0] = sum of the liquid mask, scalars[1] = loss; writes dL/dout into grad.
 int net_loss(hipStream_t s, const float* act, const float* target, float* grad, uint64_t nt, float* partial,
              float* scalars);
-// Backward pass: grad must be zero except dL/dout at kActOut; writes every parameter gradient and
-// leaves dL/dinput at kActIn of each gradient record.
-int net_backward(hipStream_t s, const float* params, const float* act, float* grad, uint64_t nt, float* partial,
+// Backward pass of the last net_forward (its packed weights): grad must be zero except dL/dout at kActOut;
+// writes every parameter gradient and leaves dL/dinput at kActIn of each gradient record.
+constexpr uint64_t kGradChunks = 512;  // tile chunks with partial parameter gradients of their own
+int net_backward(hipStream_t s, const float* packed, const float* act, float* grad, uint64_t nt, float* partial,
                  uint64_t partial_floats, float* grad_params);
 int net_clear(hipStream_t s, float* p, uint64_t n);
 int net_adam(hipStream_t s, float* w, const float* g, float* m1, float* m2, uint64_t n, float lr, int step);

@@ -51,133 +51,210 @@ __device__ inline void tap(int k, int& dz, int& dy, int& dx) {
   dx = k % 3 - 1;
 }
 
-// y[co][v] = relu?(b[co] + sum_{ci,k} w[co][ci][k] x[ci][v + off(k)]), x = a-channels ++ b-channels.
-template <int COUT>
-__global__ void k_conv_fwd(float* act, uint64_t ntiles, LayerSpec L, const float* w, const float* bias) {
-  const int s = L.side, n = s * s * s;
-  const uint64_t gid = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  if (gid >= ntiles * uint64_t(n)) return;
-  const uint64_t t = gid / uint64_t(n);
-  const int v = static_cast<int>(gid % uint64_t(n));
-  const int z = v / (s * s), y = (v / s) % s, x = v % s;
-  float* base = act + t * kActFloats;
-  float acc[COUT];
-#pragma unroll
-  for (int co = 0; co < COUT; ++co) acc[co] = bias[co];
-  const int cin = L.ca + L.cb;
-  for (int ci = 0; ci < cin; ++ci) {
-    const float* src = ci < L.ca ? base + L.a + ci * n : base + L.b + (ci - L.ca) * n;
-    for (int k = 0; k < 27; ++k) {
-      int dz, dy, dx;
-      tap(k, dz, dy, dx);
-      const int zz = z + dz, yy = y + dy, xx = x + dx;
-      if (zz < 0 || zz >= s || yy < 0 || yy >= s || xx < 0 || xx >= s) continue;
-      const float xv = src[(zz * s + yy) * s + xx];
-      const float* wk = w + ci * 27 + k;
-#pragma unroll
-      for (int co = 0; co < COUT; ++co) acc[co] = fmaf(wk[co * cin * 27], xv, acc[co]);
-    }
-  }
-  float* dst = base + L.y;
-#pragma unroll
-  for (int co = 0; co < COUT; ++co) dst[co * n + v] = (L.relu && acc[co] < 0.f) ? 0.f : acc[co];
-}
+// ---- FP32 convolutions (training) ----
+// A 3x3x3 convolution of zero-padded cubes as a register tile: a lane holds VX voxels of one row and CO
+// output channels, reads VX + 2 values per input row from LDS and feeds 3 VX CO multiply-adds from them,
+// the weights coming as wave-uniform scalars (packed [group][input][tap][CO], so an input's 27 CO weights
+// are a few wide scalar loads). Inputs are staged CC channels at a time with a one-voxel zero halo, which takes the place
+// of the bounds tests. Bound by FP32 issue: 48 multiply-adds per two LDS reads of a row. The backward
+// pass of the data is the same convolution of the output gradient with the taps mirrored and the
+// channels exchanged. With one lane per voxel and input, taps tested against the cube's faces and weights
+// read one by one, loss and gradients of 512 tiles took 11.2 ms (the weights' gradients, one lane per weight
+// over whole tiles, half of it); now 1.85 ms, 1.35 ms of it kernels.
+template <int SIDE>
+struct Cube {
+  static constexpr int kVoxels = SIDE * SIDE * SIDE;
+  static constexpr int kVx = SIDE < 4 ? SIDE : 4;              // voxels per lane, along x
+  static constexpr int kRows = SIDE * SIDE * (SIDE / kVx);     // lanes per tile and channel group
+  static constexpr int kTiles = kRows < 64 ? 64 / kRows : 1;   // tiles per workgroup
+  static constexpr int kRowWaves = kRows < 64 ? 1 : kRows / 64;
+  static constexpr int kPitch = SIDE == 8 ? 12 : (SIDE == 4 ? 8 : 4);  // x at index x + 1
+  static constexpr int kPlane = (SIDE + 2) * kPitch;
+  static constexpr int kPadded = (SIDE + 2) * kPlane;
+};
+constexpr int kStageChannels = 4;
 
-// dL/dx for one convolution: dx[ci][v] (+)= sum_{co,k} w[co][ci][k] g[co][v - off(k)], where g (at the
-// layer's output offset in `grad`) already includes the ReLU derivative. a-channels and b-channels of
-// the input gradient are added to what is there (both gradients of a skip tensor meet by addition).
-template <int CIN>
-__global__ void k_conv_bwd_data(float* grad, uint64_t ntiles, LayerSpec L, const float* w) {
-  const int s = L.side, n = s * s * s;
-  const uint64_t gid = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  if (gid >= ntiles * uint64_t(n)) return;
-  const uint64_t t = gid / uint64_t(n);
-  const int v = static_cast<int>(gid % uint64_t(n));
-  const int z = v / (s * s), y = (v / s) % s, x = v % s;
-  float* base = grad + t * kActFloats;
-  float acc[CIN];
-#pragma unroll
-  for (int ci = 0; ci < CIN; ++ci) acc[ci] = 0.f;
-  for (int co = 0; co < L.cout; ++co) {
-    const float* gy = base + L.y + co * n;
-    for (int k = 0; k < 27; ++k) {
-      int dz, dy, dx;
-      tap(k, dz, dy, dx);
-      const int zz = z - dz, yy = y - dy, xx = x - dx;
-      if (zz < 0 || zz >= s || yy < 0 || yy >= s || xx < 0 || xx >= s) continue;
-      const float gv = gy[(zz * s + yy) * s + xx];
-      const float* wk = w + co * CIN * 27 + k;
-#pragma unroll
-      for (int ci = 0; ci < CIN; ++ci) acc[ci] = fmaf(wk[ci * 27], gv, acc[ci]);
-    }
-  }
-#pragma unroll
-  for (int ci = 0; ci < CIN; ++ci) {
-    float* d = ci < L.ca ? base + L.a + ci * n : base + L.b + (ci - L.ca) * n;
-    d[v] += acc[ci];
-  }
-}
+// Where a convolution reads and writes in the tile records: ca channels at a, then the rest at b.
+struct ConvSpan {
+  int a, ca, b;
+  __host__ __device__ int offset(int c, int voxels) const { return c < ca ? a + c * voxels : b + (c - ca) * voxels; }
+};
 
-// Per-chunk partial gradients of one layer's weights and biases: lane (chunk, j), j < weights is
-// w[co][ci][k], j >= weights the bias of co = j - weights. Tiles of a chunk are summed in order.
-__global__ void k_conv_bwd_w(const float* act, const float* grad, uint64_t ntiles, uint64_t chunk, LayerSpec L,
-                             uint64_t nw, float* partial) {
-  const uint64_t per = nw + L.cout;
-  const uint64_t gid = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  const uint64_t nchunks = (ntiles + chunk - 1) / chunk;
-  if (gid >= per * nchunks) return;
-  const uint64_t c = gid / per, j = gid % per;
-  const int s = L.side, n = s * s * s, cin = L.ca + L.cb;
-  const uint64_t t0 = c * chunk, t1 = std::min<uint64_t>(ntiles, t0 + chunk);
-  float acc = 0.f;
-  if (j >= nw) {
-    const int co = static_cast<int>(j - nw);
-    for (uint64_t t = t0; t < t1; ++t) {
-      const float* g = grad + t * kActFloats + L.y + co * n;
-      for (int v = 0; v < n; ++v) acc += g[v];
+// kBackward: src is the gradient record (masked by act > 0 where the layer has a ReLU), results are added to
+// dst; otherwise dst = relu?(bias + sum).
+template <int SIDE, int OUT, int CO, bool kBackward>
+__global__ __launch_bounds__(64 * Cube<SIDE>::kRowWaves * (OUT / CO)) void k_conv(
+    const float* __restrict__ src, const float* __restrict__ act, float* dst, uint64_t ntiles, int cin, ConvSpan in,
+    ConvSpan out, bool relu, const float* __restrict__ w, const float* __restrict__ bias) {
+  using C = Cube<SIDE>;
+  constexpr int kThreadsHere = 64 * C::kRowWaves * (OUT / CO);
+  constexpr int kStaged = kStageChannels * C::kTiles * C::kPadded;
+  __shared__ float xs[kStaged];
+  const int tid = static_cast<int>(threadIdx.x), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave / C::kRowWaves;  // output channels [group * CO, group * CO + CO)
+  const int row = (wave % C::kRowWaves) * 64 + (tid & 63);
+  const int sub = C::kTiles > 1 ? row / C::kRows : 0, r = row % C::kRows;
+  constexpr int kPerRow = SIDE / C::kVx;
+  const int x0 = (r % kPerRow) * C::kVx, y = (r / kPerRow) % SIDE, z = r / (kPerRow * SIDE);
+  const uint64_t first = uint64_t(blockIdx.x) * C::kTiles;
+  for (int i = tid; i < kStaged; i += kThreadsHere) xs[i] = 0.f;
+  float acc[CO][C::kVx];
+#pragma unroll
+  for (int co = 0; co < CO; ++co)
+#pragma unroll
+    for (int v = 0; v < C::kVx; ++v) acc[co][v] = kBackward ? 0.f : bias[group * CO + co];
+  const float* wg = w + group * cin * 27 * CO;
+  for (int c0 = 0; c0 < cin; c0 += kStageChannels) {
+    const int cc = min(kStageChannels, cin - c0);
+    __syncthreads();
+    for (int i = tid; i < cc * C::kTiles * C::kVoxels; i += kThreadsHere) {
+      const int v = i % C::kVoxels, q = i / C::kVoxels, t = q % C::kTiles, c = q / C::kTiles;
+      if (first + t >= ntiles) continue;
+      const uint64_t at = (first + t) * kActFloats + in.offset(c0 + c, C::kVoxels) + v;
+      float value = src[at];
+      if (kBackward && relu && !(act[at] > 0.f)) value = 0.f;
+      xs[(c * C::kTiles + t) * C::kPadded + (v / (SIDE * SIDE) + 1) * C::kPlane + ((v / SIDE) % SIDE + 1) * C::kPitch +
+         v % SIDE + 1] = value;
     }
-  } else {
-    const int co = static_cast<int>(j / (uint64_t(cin) * 27));
-    const int ci = static_cast<int>((j / 27) % cin);
-    const int k = static_cast<int>(j % 27);
-    int dz, dy, dx;
-    tap(k, dz, dy, dx);
-    for (uint64_t t = t0; t < t1; ++t) {
-      const float* g = grad + t * kActFloats + L.y + co * n;
-      const float* xs = act + t * kActFloats + (ci < L.ca ? L.a + ci * n : L.b + (ci - L.ca) * n);
-      for (int z = 0; z < s; ++z) {
-        const int zz = z + dz;
-        if (zz < 0 || zz >= s) continue;
-        for (int y = 0; y < s; ++y) {
-          const int yy = y + dy;
-          if (yy < 0 || yy >= s) continue;
-          for (int x = 0; x < s; ++x) {
-            const int xx = x + dx;
-            if (xx < 0 || xx >= s) continue;
-            acc = fmaf(g[(z * s + y) * s + x], xs[(zz * s + yy) * s + xx], acc);
-          }
-        }
+    __syncthreads();
+    for (int c = 0; c < cc; ++c) {
+      const float* base = xs + (c * C::kTiles + sub) * C::kPadded + z * C::kPlane + y * C::kPitch + x0;
+      const float* wc = wg + (c0 + c) * 27 * CO;
+#pragma unroll
+      for (int k = 0; k < 9; ++k) {
+        float x[C::kVx + 2];
+#pragma unroll
+        for (int v = 0; v < C::kVx + 2; ++v) x[v] = base[(k / 3) * C::kPlane + (k % 3) * C::kPitch + v];
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+          for (int co = 0; co < CO; ++co)
+#pragma unroll
+            for (int v = 0; v < C::kVx; ++v) acc[co][v] = fmaf(wc[(k * 3 + dx) * CO + co], x[v + dx], acc[co][v]);
       }
     }
   }
-  partial[c * per + j] = acc;
+  if (first + sub >= ntiles) return;
+#pragma unroll
+  for (int co = 0; co < CO; ++co) {
+    float* d = dst + (first + sub) * kActFloats + out.offset(group * CO + co, C::kVoxels) + (z * SIDE + y) * SIDE + x0;
+#pragma unroll
+    for (int v = 0; v < C::kVx; ++v) {
+      if (kBackward) d[v] += acc[co][v];
+      else d[v] = relu && acc[co][v] < 0.f ? 0.f : acc[co][v];
+    }
+  }
 }
 
-// out[j] = sum over chunks in order (deterministic).
-__global__ void k_reduce_chunks(const float* partial, uint64_t nchunks, uint64_t per, float* out) {
-  const uint64_t j = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  if (j >= per) return;
+// Output channels per lane of k_conv, forward and data backward: four on the 8^3 layers, two on the smaller
+// cubes, whose few voxels would leave the chip idle with more.
+constexpr int kForwardCo[kNetLayers] = {4, 4, 2, 2, 2, 2, 2, 2, 4, 1};
+constexpr int kBackwardCo[kNetLayers] = {2, 4, 1, 2, 2, 2, 4, 2, 6, 4};
+
+// The layers' weights [co][ci][k] packed for k_conv: forward [co / CO][ci][k][co % CO], and for the data's
+// backward pass [ci / CO][co][k'][ci % CO] with the taps mirrored (k' = 26 - k).
+struct PackSpec {
+  int first[kNetLayers + 1], cin[kNetLayers], cout[kNetLayers], fco[kNetLayers], bco[kNetLayers];
+};
+__global__ void k_pack_weights(const float* params, PackSpec spec, float* forward, float* backward) {
+  const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i >= spec.first[kNetLayers]) return;
+  int l = 0;
+  while (i >= spec.first[l + 1]) ++l;
+  const int cin = spec.cin[l], cout = spec.cout[l], nw = cin * cout * 27, j = i - spec.first[l];
+  if (j >= nw) return;  // biases are read in place
+  const int co = j / (cin * 27), ci = (j / 27) % cin, k = j % 27, f = spec.fco[l], b = spec.bco[l];
+  forward[spec.first[l] + ((co / f * cin + ci) * 27 + k) * f + co % f] = params[i];
+  backward[spec.first[l] + ((ci / b * cout + co) * 27 + 26 - k) * b + ci % b] = params[i];
+}
+
+// Per-chunk partial gradients of one layer's weights (w[co][ci][k]) and biases, tiles of a chunk in order.
+// A lane owns one input channel and row offset (ci, kz, ky) with its three x taps for all COUT outputs; it
+// walks the tile's rows, its own input row coming from padded LDS and the output gradients (masked by the
+// ReLU) as LDS broadcasts: 3 COUT multiply-adds per voxel for COUT / 4 broadcast reads. One more lane reads a
+// row of ones: its middle tap is the bias gradient. Bound by FP32 issue.
+template <int SIDE, int COUT, int CI>
+__global__ __launch_bounds__((CI * 9 + 1 + 63) / 64 * 64) void k_conv_grad(const float* __restrict__ act,
+                                                                           const float* __restrict__ grad,
+                                                                           uint64_t ntiles, uint64_t chunk, int cin,
+                                                                           ConvSpan in, int y_offset, bool relu,
+                                                                           float* partial) {
+  constexpr int kSide2 = SIDE + 2, kVoxels = SIDE * SIDE * SIDE, kPadded = kSide2 * kSide2 * kSide2;
+  constexpr int kLanes = (CI * 9 + 1 + 63) / 64 * 64;
+  __shared__ float xs[CI * kPadded];
+  __shared__ __attribute__((aligned(16))) float gs[kVoxels * COUT];
+  const int tid = static_cast<int>(threadIdx.x), c0 = static_cast<int>(blockIdx.y) * CI;
+  const int ci = tid / 9, kz = (tid % 9) / 3, ky = tid % 3;
+  const bool bias = tid == CI * 9, used = tid < CI * 9 && c0 + ci < cin;
+  float acc[3][COUT];
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int co = 0; co < COUT; ++co) acc[d][co] = 0.f;
+  for (int i = tid; i < CI * kPadded; i += kLanes) xs[i] = 0.f;
+  const uint64_t t0 = uint64_t(blockIdx.x) * chunk, t1 = t0 + chunk < ntiles ? t0 + chunk : ntiles;
+  const float* row0 = xs + (used ? ci : 0) * kPadded + (used ? kz * kSide2 * kSide2 + ky * kSide2 : 0);
+  for (uint64_t t = t0; t < t1; ++t) {
+    __syncthreads();
+    const float* rec = act + t * kActFloats;
+    for (int i = tid; i < CI * kVoxels; i += kLanes) {
+      const int c = i / kVoxels, v = i % kVoxels;
+      if (c0 + c >= cin) continue;
+      xs[c * kPadded + ((v / (SIDE * SIDE) + 1) * kSide2 + (v / SIDE) % SIDE + 1) * kSide2 + v % SIDE + 1] =
+          rec[in.offset(c0 + c, kVoxels) + v];
+    }
+    for (int i = tid; i < COUT * kVoxels; i += kLanes) {
+      const int v = i % kVoxels, co = i / kVoxels;
+      const float g = grad[t * kActFloats + y_offset + i];
+      gs[v * COUT + co] = relu && !(rec[y_offset + i] > 0.f) ? 0.f : g;
+    }
+    __syncthreads();
+    for (int zy = 0; zy < SIDE * SIDE; ++zy) {
+      const float* p = row0 + (zy / SIDE) * kSide2 * kSide2 + (zy % SIDE) * kSide2;
+      float x[kSide2];
+#pragma unroll
+      for (int v = 0; v < kSide2; ++v) x[v] = bias ? 1.f : p[v];
+#pragma unroll
+      for (int v = 0; v < SIDE; ++v) {
+        const float* g = gs + (zy * SIDE + v) * COUT;
+#pragma unroll
+        for (int co = 0; co < COUT; ++co)
+#pragma unroll
+          for (int d = 0; d < 3; ++d) acc[d][co] = fmaf(g[co], x[v + d], acc[d][co]);
+      }
+    }
+  }
+  const int nw = COUT * cin * 27;
+  float* out = partial + uint64_t(blockIdx.x) * (nw + COUT);
+  if (used) {
+#pragma unroll
+    for (int co = 0; co < COUT; ++co)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) out[(co * cin + c0 + ci) * 27 + (kz * 3 + ky) * 3 + d] = acc[d][co];
+  } else if (bias && c0 == 0) {
+#pragma unroll
+    for (int co = 0; co < COUT; ++co) out[nw + co] = acc[1][co];
+  }
+}
+
+// out[j] = sum over chunks: sixteen lanes take a run of chunks each, their sums are added in order
+// (deterministic). The runs are short so that their dependent loads are: one lane over 256 chunks took
+// 61 us a layer.
+constexpr int kReduceOutputs = 16, kReduceRuns = 16;
+__global__ __launch_bounds__(kReduceOutputs * kReduceRuns) void k_reduce_chunks(const float* partial, uint64_t nchunks,
+                                                                                uint64_t per, float* out) {
+  __shared__ float red[kReduceRuns][kReduceOutputs];
+  const int o = static_cast<int>(threadIdx.x) % kReduceOutputs, run = static_cast<int>(threadIdx.x) / kReduceOutputs;
+  const uint64_t j = blockIdx.x * uint64_t(kReduceOutputs) + o;
+  const uint64_t c0 = nchunks * run / kReduceRuns, c1 = nchunks * (run + 1) / kReduceRuns;
   float a = 0.f;
-  for (uint64_t c = 0; c < nchunks; ++c) a += partial[c * per + j];
+  if (j < per)
+    for (uint64_t c = c0; c < c1; ++c) a += partial[c * per + j];
+  red[run][o] = a;
+  __syncthreads();
+  if (run != 0 || j >= per) return;
+  for (int r = 1; r < kReduceRuns; ++r) a += red[r][o];
   out[j] = a;
-}
-
-__global__ void k_relu_bwd(const float* act, float* grad, uint64_t ntiles, int off, int count) {
-  const uint64_t gid = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x;
-  if (gid >= ntiles * uint64_t(count)) return;
-  const uint64_t t = gid / uint64_t(count);
-  const uint64_t i = t * kActFloats + off + gid % uint64_t(count);
-  if (!(act[i] > 0.f)) grad[i] = 0.f;
 }
 
 // 2x2x2 average pooling from side 2h to side h (fwd), and its adjoint added into the input gradient.
@@ -573,44 +650,93 @@ __global__ __launch_bounds__(256) void k_unet_infer(float* act, const bf16x4* fr
   conv_lds<9, kA8, 8, 0, 4, 0>(lds, frags, params, rec + kActOut);
 }
 
-template <int N>
-void conv_fwd_n(hipStream_t s, float* act, uint64_t nt, const LayerSpec& L, const float* w, const float* b) {
-  const uint64_t lanes = nt * uint64_t(L.side * L.side * L.side);
-  k_conv_fwd<N><<<grid_for(lanes), kThreads, 0, s>>>(act, nt, L, w, b);
-}
-template <int N>
-void conv_bwd_n(hipStream_t s, float* grad, uint64_t nt, const LayerSpec& L, const float* w) {
-  const uint64_t lanes = nt * uint64_t(L.side * L.side * L.side);
-  k_conv_bwd_data<N><<<grid_for(lanes), kThreads, 0, s>>>(grad, nt, L, w);
+template <int SIDE, int OUT, int CO, bool kBackward>
+void conv_n(hipStream_t s, const float* src, const float* act, float* dst, uint64_t nt, int cin, const ConvSpan& in,
+            const ConvSpan& out, bool relu, const float* w, const float* bias) {
+  using C = Cube<SIDE>;
+  k_conv<SIDE, OUT, CO, kBackward>
+      <<<static_cast<unsigned>((nt + C::kTiles - 1) / C::kTiles), 64 * C::kRowWaves * (OUT / CO), 0, s>>>(
+          src, act, dst, nt, cin, in, out, relu, w, bias);
 }
 
-int conv_fwd(hipStream_t s, float* act, uint64_t nt, int l, const float* params) {
+int conv_fwd(hipStream_t s, float* act, uint64_t nt, int l, const float* params, const float* packed) {
   const LayerSpec& L = kLayers[l];
-  const float* w = params + layer_offset(l);
-  const float* b = w + layer_weights(l);
-  switch (L.cout) {
-    case 1: conv_fwd_n<1>(s, act, nt, L, w, b); break;
-    case 8: conv_fwd_n<8>(s, act, nt, L, w, b); break;
-    case 16: conv_fwd_n<16>(s, act, nt, L, w, b); break;
-    case 32: conv_fwd_n<32>(s, act, nt, L, w, b); break;
+  const float* w = packed + layer_offset(l);
+  const float* b = params + layer_offset(l) + layer_weights(l);
+  const ConvSpan in{L.a, L.ca, L.b}, out{L.y, L.cout, 0};
+  const int cin = L.ca + L.cb;
+  switch (L.side * 100 + L.cout) {
+    case 801: conv_n<8, 1, kForwardCo[9], false>(s, act, act, act, nt, cin, in, out, L.relu, w, b); break;
+    case 808: conv_n<8, 8, kForwardCo[0], false>(s, act, act, act, nt, cin, in, out, L.relu, w, b); break;
+    case 416: conv_n<4, 16, kForwardCo[2], false>(s, act, act, act, nt, cin, in, out, L.relu, w, b); break;
+    case 232: conv_n<2, 32, kForwardCo[4], false>(s, act, act, act, nt, cin, in, out, L.relu, w, b); break;
     default: return FL_INTERNAL;
   }
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
 
-int conv_bwd_data(hipStream_t s, float* grad, uint64_t nt, int l, const float* params) {
+int conv_bwd_data(hipStream_t s, const float* act, float* grad, uint64_t nt, int l, const float* packed) {
   const LayerSpec& L = kLayers[l];
-  const float* w = params + layer_offset(l);
-  switch (L.ca + L.cb) {
-    case 4: conv_bwd_n<4>(s, grad, nt, L, w); break;
-    case 8: conv_bwd_n<8>(s, grad, nt, L, w); break;
-    case 16: conv_bwd_n<16>(s, grad, nt, L, w); break;
-    case 24: conv_bwd_n<24>(s, grad, nt, L, w); break;
-    case 32: conv_bwd_n<32>(s, grad, nt, L, w); break;
-    case 48: conv_bwd_n<48>(s, grad, nt, L, w); break;
+  const float* w = packed + layer_offset(kNetLayers) + layer_offset(l);
+  const ConvSpan in{L.y, L.cout, 0}, out{L.a, L.ca, L.b};
+  const auto run = [&](auto conv) { conv(s, grad, act, grad, nt, L.cout, in, out, L.relu, w, nullptr); };
+  switch (L.side * 100 + L.ca + L.cb) {
+    case 804: run(conv_n<8, 4, kBackwardCo[0], true>); break;
+    case 808: run(conv_n<8, 8, kBackwardCo[1], true>); break;
+    case 824: run(conv_n<8, 24, kBackwardCo[8], true>); break;
+    case 408: run(conv_n<4, 8, kBackwardCo[2], true>); break;
+    case 416: run(conv_n<4, 16, kBackwardCo[3], true>); break;
+    case 448: run(conv_n<4, 48, kBackwardCo[6], true>); break;
+    case 216: run(conv_n<2, 16, kBackwardCo[4], true>); break;
+    case 232: run(conv_n<2, 32, kBackwardCo[5], true>); break;
     default: return FL_INTERNAL;
   }
+  FL_HIP(hipGetLastError());
+  return FL_OK;
+}
+
+template <int SIDE, int COUT, int CI>
+void grad_n(hipStream_t s, const float* act, const float* grad, uint64_t nt, uint64_t chunk, const LayerSpec& L,
+            float* partial) {
+  const int cin = L.ca + L.cb;
+  const dim3 grid(static_cast<unsigned>((nt + chunk - 1) / chunk), static_cast<unsigned>((cin + CI - 1) / CI));
+  k_conv_grad<SIDE, COUT, CI><<<grid, (CI * 9 + 1 + 63) / 64 * 64, 0, s>>>(act, grad, nt, chunk, cin,
+                                                                           ConvSpan{L.a, L.ca, L.b}, L.y, L.relu, partial);
+}
+
+// Input channels per workgroup: as many as fill two to four waves with nine rows each and leave room in
+// LDS for two workgroups on a CU.
+int conv_bwd_weights(hipStream_t s, const float* act, const float* grad, uint64_t nt, uint64_t chunk, int l,
+                     float* partial) {
+  const LayerSpec& L = kLayers[l];
+  const int cin = L.ca + L.cb;
+  if (L.side == 8 && L.cout == 1) grad_n<8, 1, 8>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 8 && cin == 24) grad_n<8, 8, 12>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 8 && cin == 8) grad_n<8, 8, 8>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 8 && cin == 4) grad_n<8, 8, 4>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 4 && cin == 48) grad_n<4, 16, 24>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 4 && cin == 16) grad_n<4, 16, 16>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 4 && cin == 8) grad_n<4, 16, 8>(s, act, grad, nt, chunk, L, partial);
+  else if (L.side == 2) grad_n<2, 32, 16>(s, act, grad, nt, chunk, L, partial);
+  else return FL_INTERNAL;
+  FL_HIP(hipGetLastError());
+  return FL_OK;
+}
+
+// Both packings of the weights: packed holds 2 * net_param_count() floats.
+int pack_weights(hipStream_t s, const float* params, float* packed) {
+  PackSpec spec{};
+  for (int l = 0; l < kNetLayers; ++l) {
+    spec.first[l] = static_cast<int>(layer_offset(l));
+    spec.cin[l] = kLayers[l].ca + kLayers[l].cb;
+    spec.cout[l] = kLayers[l].cout;
+    spec.fco[l] = kForwardCo[l];
+    spec.bco[l] = kBackwardCo[l];
+  }
+  spec.first[kNetLayers] = static_cast<int>(layer_offset(kNetLayers));
+  k_pack_weights<<<grid_for(spec.first[kNetLayers]), kThreads, 0, s>>>(params, spec, packed,
+                                                                      packed + layer_offset(kNetLayers));
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
@@ -619,22 +745,23 @@ int conv_bwd_data(hipStream_t s, float* grad, uint64_t nt, int l, const float* p
 
 uint64_t net_param_count() { return layer_offset(kNetLayers); }
 
-int net_forward(hipStream_t s, const float* params, float* act, uint64_t nt) {
+int net_forward(hipStream_t s, const float* params, float* packed, float* act, uint64_t nt) {
   if (!nt) return FL_OK;
-  FL_TRY(conv_fwd(s, act, nt, 0, params));
-  FL_TRY(conv_fwd(s, act, nt, 1, params));
+  FL_TRY(pack_weights(s, params, packed));
+  FL_TRY(conv_fwd(s, act, nt, 0, params, packed));
+  FL_TRY(conv_fwd(s, act, nt, 1, params, packed));
   k_pool_fwd<<<grid_for(nt * 8 * 64), kThreads, 0, s>>>(act, nt, 8, 4, kActA1, kActP1);
-  FL_TRY(conv_fwd(s, act, nt, 2, params));
-  FL_TRY(conv_fwd(s, act, nt, 3, params));
+  FL_TRY(conv_fwd(s, act, nt, 2, params, packed));
+  FL_TRY(conv_fwd(s, act, nt, 3, params, packed));
   k_pool_fwd<<<grid_for(nt * 16 * 8), kThreads, 0, s>>>(act, nt, 16, 2, kActA3, kActP2);
-  FL_TRY(conv_fwd(s, act, nt, 4, params));
-  FL_TRY(conv_fwd(s, act, nt, 5, params));
+  FL_TRY(conv_fwd(s, act, nt, 4, params, packed));
+  FL_TRY(conv_fwd(s, act, nt, 5, params, packed));
   k_up_fwd<<<grid_for(nt * 32 * 64), kThreads, 0, s>>>(act, nt, 32, 2, kActA5, kActU5);
-  FL_TRY(conv_fwd(s, act, nt, 6, params));
-  FL_TRY(conv_fwd(s, act, nt, 7, params));
+  FL_TRY(conv_fwd(s, act, nt, 6, params, packed));
+  FL_TRY(conv_fwd(s, act, nt, 7, params, packed));
   k_up_fwd<<<grid_for(nt * 16 * 512), kThreads, 0, s>>>(act, nt, 16, 4, kActA7, kActU7);
-  FL_TRY(conv_fwd(s, act, nt, 8, params));
-  FL_TRY(conv_fwd(s, act, nt, 9, params));
+  FL_TRY(conv_fwd(s, act, nt, 8, params, packed));
+  FL_TRY(conv_fwd(s, act, nt, 9, params, packed));
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
@@ -660,58 +787,44 @@ int net_infer(hipStream_t s, const float* params, void* frags, float* act, uint6
   return FL_OK;
 }
 
-int net_backward(hipStream_t s, const float* params, const float* act, float* grad, uint64_t nt, float* partial,
+int net_backward(hipStream_t s, const float* packed, const float* act, float* grad, uint64_t nt, float* partial,
                  uint64_t partial_floats, float* grad_params) {
   if (!nt) return FL_OK;
-  const uint64_t chunk = 8, nchunks = (nt + chunk - 1) / chunk;
+  const uint64_t chunk = (nt + kGradChunks - 1) / kGradChunks, nchunks = (nt + chunk - 1) / chunk;
   auto weights = [&](int l) -> int {
     const LayerSpec& L = kLayers[l];
-    const uint64_t nw = layer_weights(l), per = nw + L.cout;
+    const uint64_t per = layer_weights(l) + L.cout;
     if (per * nchunks > partial_floats) return FL_RESOURCE_EXHAUSTED;
-    k_conv_bwd_w<<<grid_for(per * nchunks), kThreads, 0, s>>>(act, grad, nt, chunk, L, nw, partial);
-    k_reduce_chunks<<<grid_for(per), kThreads, 0, s>>>(partial, nchunks, per, grad_params + layer_offset(l));
+    FL_TRY(conv_bwd_weights(s, act, grad, nt, chunk, l, partial));
+    k_reduce_chunks<<<grid_for(per, kReduceOutputs), kReduceOutputs * kReduceRuns, 0, s>>>(partial, nchunks, per, grad_params + layer_offset(l));
     FL_HIP(hipGetLastError());
     return FL_OK;
   };
-  auto relu = [&](int l) {
-    const LayerSpec& L = kLayers[l];
-    const int count = L.cout * L.side * L.side * L.side;
-    k_relu_bwd<<<grid_for(nt * count), kThreads, 0, s>>>(act, grad, nt, L.y, count);
-  };
   // Layer 9 (linear), 8, up7, 7, 6, up5, 5, 4, pool2, 3, 2, pool1, 1, 0.
   FL_TRY(weights(9));
-  FL_TRY(conv_bwd_data(s, grad, nt, 9, params));
-  relu(8);
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 9, packed));
   FL_TRY(weights(8));
-  FL_TRY(conv_bwd_data(s, grad, nt, 8, params));
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 8, packed));
   k_up_bwd<<<grid_for(nt * 16 * 64), kThreads, 0, s>>>(grad, nt, 16, 4, kActA7, kActU7);
-  relu(7);
   FL_TRY(weights(7));
-  FL_TRY(conv_bwd_data(s, grad, nt, 7, params));
-  relu(6);
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 7, packed));
   FL_TRY(weights(6));
-  FL_TRY(conv_bwd_data(s, grad, nt, 6, params));
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 6, packed));
   k_up_bwd<<<grid_for(nt * 32 * 8), kThreads, 0, s>>>(grad, nt, 32, 2, kActA5, kActU5);
-  relu(5);
   FL_TRY(weights(5));
-  FL_TRY(conv_bwd_data(s, grad, nt, 5, params));
-  relu(4);
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 5, packed));
   FL_TRY(weights(4));
-  FL_TRY(conv_bwd_data(s, grad, nt, 4, params));
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 4, packed));
   k_pool_bwd<<<grid_for(nt * 16 * 64), kThreads, 0, s>>>(grad, nt, 16, 2, kActA3, kActP2);
-  relu(3);
   FL_TRY(weights(3));
-  FL_TRY(conv_bwd_data(s, grad, nt, 3, params));
-  relu(2);
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 3, packed));
   FL_TRY(weights(2));
-  FL_TRY(conv_bwd_data(s, grad, nt, 2, params));
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 2, packed));
   k_pool_bwd<<<grid_for(nt * 8 * 512), kThreads, 0, s>>>(grad, nt, 8, 4, kActA1, kActP1);
-  relu(1);
   FL_TRY(weights(1));
-  FL_TRY(conv_bwd_data(s, grad, nt, 1, params));
-  relu(0);
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 1, packed));
   FL_TRY(weights(0));
-  FL_TRY(conv_bwd_data(s, grad, nt, 0, params));  // input gradient, for checks
+  FL_TRY(conv_bwd_data(s, act, grad, nt, 0, packed));  // input gradient, for checks
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
@@ -806,6 +919,7 @@ void destroy_learn(fl_ctx* ctx) {
   lfree(L->data_in);
   lfree(L->data_target);
   lfree(L->frags);
+  lfree(L->packed);
   delete L;
   ctx->learn = nullptr;
 }
@@ -825,10 +939,10 @@ int train_epoch(fl_ctx* ctx, uint64_t batch, float lr, uint64_t seed, float* mea
     FL_HIP(hipMemcpyAsync(L->batch_index, order.data() + b0, nt * sizeof(int32_t), hipMemcpyHostToDevice, s));
     k_load_batch<<<grid_for(nt * 2560), kThreads, 0, s>>>(L->data_in, L->data_target, L->batch_index, nt, L->act,
                                                           L->batch_target);
-    FL_TRY(net_forward(s, L->params, L->act, nt));
+    FL_TRY(net_forward(s, L->params, L->packed, L->act, nt));
     FL_TRY(net_clear(s, L->grad, nt * kActFloats));
     FL_TRY(net_loss(s, L->act, L->batch_target, L->grad, nt, L->partial, L->scalars));
-    FL_TRY(net_backward(s, L->params, L->act, L->grad, nt, L->partial, L->partial_floats, L->gparams));
+    FL_TRY(net_backward(s, L->packed, L->act, L->grad, nt, L->partial, L->partial_floats, L->gparams));
     FL_TRY(net_adam(s, L->params, L->gparams, L->m1, L->m2, L->np, lr, ++L->step));
     float h[2];
     FL_HIP(hipMemcpyAsync(h, L->scalars, 2 * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -853,7 +967,7 @@ int eval_pairs(fl_ctx* ctx, uint64_t batch, float* mean_loss) {
     FL_HIP(hipMemcpyAsync(L->batch_index, order.data() + b0, nt * sizeof(int32_t), hipMemcpyHostToDevice, s));
     k_load_batch<<<grid_for(nt * 2560), kThreads, 0, s>>>(L->data_in, L->data_target, L->batch_index, nt, L->act,
                                                           L->batch_target);
-    FL_TRY(net_forward(s, L->params, L->act, nt));
+    FL_TRY(net_forward(s, L->params, L->packed, L->act, nt));
     FL_TRY(net_clear(s, L->grad, nt * kActFloats));
     FL_TRY(net_loss(s, L->act, L->batch_target, L->grad, nt, L->partial, L->scalars));
     float h[2];
@@ -885,7 +999,7 @@ int fl_learn_setup(fl_ctx* ctx, uint64_t tile_capacity, uint64_t pair_capacity) 
   L->tile_cap = tile_capacity;
   L->data_cap = pair_capacity;
   const uint64_t train_tiles = std::min<uint64_t>(tile_capacity, 1024);
-  L->partial_floats = std::max<uint64_t>(27680 * ((train_tiles + 7) / 8), 2 * tile_capacity + 1024);
+  L->partial_floats = std::max<uint64_t>(27680 * std::min<uint64_t>(train_tiles, fl::kGradChunks), 2 * tile_capacity + 1024);
   int st = FL_OK;
   auto A = [&](auto** p, uint64_t n) {
     if (st == FL_OK) st = fl::lalloc(p, n);
@@ -905,6 +1019,7 @@ int fl_learn_setup(fl_ctx* ctx, uint64_t tile_capacity, uint64_t pair_capacity) 
   A(&L->data_in, pair_capacity * 2048);
   A(&L->data_target, pair_capacity * 512);
   A(&L->frags, fl::net_fragment_bytes());
+  A(&L->packed, 2 * L->np);
   if (st != FL_OK) {
     fl::destroy_learn(ctx);
     return FL_RESOURCE_EXHAUSTED;
@@ -947,7 +1062,7 @@ static int learn_forward(fl_ctx* ctx, const float* inputs, size_t n, float* outp
   if (mfma) {
     FL_TRY(fl::net_infer(s, L->params, L->frags, L->act, n));
   } else {
-    FL_TRY(fl::net_forward(s, L->params, L->act, n));
+    FL_TRY(fl::net_forward(s, L->params, L->packed, L->act, n));
   }
   fl::k_get_slot<<<fl::grid_for(n * 512), fl::kThreads, 0, s>>>(L->act, n, fl::kActOut, 512, L->stage);
   FL_HIP(hipMemcpyAsync(outputs, L->stage, n * 512 * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -973,10 +1088,10 @@ int fl_learn_loss_grad(fl_ctx* ctx, const float* inputs, const float* targets, s
   FL_HIP(hipMemcpyAsync(L->stage, inputs, n * 2048 * sizeof(float), hipMemcpyHostToDevice, s));
   FL_HIP(hipMemcpyAsync(L->batch_target, targets, n * 512 * sizeof(float), hipMemcpyHostToDevice, s));
   fl::k_put_inputs<<<fl::grid_for(n * 2048), fl::kThreads, 0, s>>>(L->stage, n, L->act);
-  FL_TRY(fl::net_forward(s, L->params, L->act, n));
+  FL_TRY(fl::net_forward(s, L->params, L->packed, L->act, n));
   FL_TRY(fl::net_clear(s, L->grad, n * fl::kActFloats));
   FL_TRY(fl::net_loss(s, L->act, L->batch_target, L->grad, n, L->partial, L->scalars));
-  FL_TRY(fl::net_backward(s, L->params, L->act, L->grad, n, L->partial, L->partial_floats, L->gparams));
+  FL_TRY(fl::net_backward(s, L->packed, L->act, L->grad, n, L->partial, L->partial_floats, L->gparams));
   float h[2];
   FL_HIP(hipMemcpyAsync(h, L->scalars, 2 * sizeof(float), hipMemcpyDeviceToHost, s));
   if (grad_params) FL_HIP(hipMemcpyAsync(grad_params, L->gparams, L->np * sizeof(float), hipMemcpyDeviceToHost, s));

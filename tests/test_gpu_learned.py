@@ -76,6 +76,41 @@ def test_network_forward_and_gradients_match_the_oracle(ctx):
     assert np.abs(gi - wi).max() <= 2e-3 * np.abs(wi).max()
 
 
+@pytest.mark.parametrize("tiles", [1, 3, 4, 15, 17])
+def test_gradients_at_partial_groups_of_tiles(ctx, tiles):
+    """Tile counts that fill the convolutions' groups (1, 4 and 16 tiles) in part, the bars of the test above."""
+    net = H.Network(ctx, tiles=32, pairs=1)
+    p = O.unet_init(5).astype(np.float32)
+    assert net.set_params(p) == H.OK
+    x, t = random_tiles(tiles, tiles)
+    x, t = x.astype(np.float32), t.astype(np.float32)
+    s, loss, gp, gi = net.loss_grad(x, t)
+    assert s == H.OK
+    wl, wg, wi = O.unet_loss_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), True)
+    assert abs(loss - wl) <= 1e-4 * abs(wl)
+    for sl in layer_slices():
+        assert np.abs(gp[sl] - wg[sl]).max() <= 2e-3 * np.abs(wg[sl]).max()
+    assert np.abs(gi - wi).max() <= 2e-3 * np.abs(wi).max()
+
+
+def test_gradients_of_many_tiles_are_the_sum_of_the_parts(ctx):
+    """600 tiles make chunks of two tiles per partial gradient: the mask-weighted gradients of two parts add up to
+    the whole's, within FP32 sums of 600 x 512 terms in another order (1e-4 of each layer's largest)."""
+    net = H.Network(ctx, tiles=1024, pairs=1)
+    assert net.set_params(O.unet_init(6).astype(np.float32)) == H.OK
+    x, t = random_tiles(600, 8)
+    x, t = x.astype(np.float32), t.astype(np.float32)
+    total, parts = x[:, 1].sum(dtype=np.float64), 0.0
+    for sel in (slice(0, 211), slice(211, 600)):
+        s, _, gp, _ = net.loss_grad(x[sel], t[sel])
+        assert s == H.OK
+        parts = parts + gp.astype(np.float64) * (x[sel, 1].sum(dtype=np.float64) / total)
+    s, _, whole, _ = net.loss_grad(x, t)
+    assert s == H.OK
+    for sl in layer_slices():
+        assert np.abs(whole[sl] - parts[sl]).max() <= 1e-4 * np.abs(whole[sl]).max()
+
+
 def test_training_lowers_the_loss(ctx):
     # Targets: a fixed linear smoothing of the residual channel, learnable by the network.
     net = H.Network(ctx, tiles=256, pairs=1024)
