@@ -659,7 +659,7 @@ int fl_reserve(fl_ctx* ctx) {
     FL_TRY(grow(&B.counts, &B.cap[13], 5));
     FL_TRY(grow(&B.phi, &B.cap[14], 9 * nc));
     FL_TRY(grow(&B.work, &B.cap[15], nc));
-    FL_TRY(grow(&B.uncut, &B.cap[16], 2));
+    FL_TRY(grow(&B.uncut, &B.cap[16], 3));
     // A sampled solid: 8 corner samples per candidate, one face velocity per owned slot.
     FL_TRY(grow(&B.solids, &B.cap[17], 8 * nc));
     FL_TRY(grow(&B.face_velocities, &B.cap[18], 192 * nb));
@@ -1034,7 +1034,8 @@ int fl_build_pressure_links(fl_ctx* ctx, const fl_frozen_view* view, const fl_pr
   const LinkDevice d{B.blocks, g.block_count, B.centers, g.center_count, B.cells, g.cell_count, B.faces, g.face_count,
                      h, g.step_duration, g.liquid_density, g.surface_tension, B.fields, B.predicted,
                      F.ambient_pressure, B.wetted, F.wetted_count, B.air, F.air_count, B.interfaces,
-                     F.interface_count};
+                     F.interface_count, fl::BlockIndex{B.blocks, g.block_count, nullptr, fl::Box{}}, {}, {}, nullptr,
+                     nullptr, nullptr};
   FL_TRY(reset_error(ctx));
   FL_TRY(build_links_device(ctx, d, nullptr, nullptr, nullptr, true));
   FL_TRY(first_error_code(ctx));
@@ -1153,7 +1154,7 @@ int fl_freeze_geometry(fl_ctx* ctx, const fl_freeze_inputs* inputs, fl_frozen_ce
   FL_TRY(grow(&B.counts, &B.cap[13], 5));
   FL_TRY(grow(&B.phi, &B.cap[14], 9 * nc_in));
   FL_TRY(grow(&B.work, &B.cap[15], nc_in));
-  FL_TRY(grow(&B.uncut, &B.cap[16], 2));
+  FL_TRY(grow(&B.uncut, &B.cap[16], 3));
   if (sampled) {
     FL_TRY(grow(&B.solids, &B.cap[17], I.solid_corner_count));
     FL_TRY(grow(&B.face_velocities, &B.cap[18], I.face_velocity_count));
@@ -1194,7 +1195,8 @@ int fl_freeze_geometry(fl_ctx* ctx, const fl_freeze_inputs* inputs, fl_frozen_ce
                        B.work,       B.uncut,
                        sampled ? static_cast<int>(I.has_sampled_solid) : 0, sampled ? B.solids : nullptr,
                        sampled ? I.solid_corner_count : 0, sampled ? B.face_velocities : nullptr,
-                       sampled ? I.face_velocity_count : 0, sampled ? B.solid_phi : nullptr};
+                       sampled ? I.face_velocity_count : 0, sampled ? B.solid_phi : nullptr,
+                       fl::BlockIndex{B.blocks, I.block_count, nullptr, fl::Box{}}, {}, {}, {}};
   const auto read_counts = [&]() -> int {
     FL_HIP(hipMemcpyAsync(ctx->host_words, B.counts, 3 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     FL_HIP(hipStreamSynchronize(s));

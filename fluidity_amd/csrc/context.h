@@ -258,6 +258,23 @@ int remap_topology(fl_ctx* ctx, const fl_block_state* pb, uint64_t pnb, const fl
                    const fl_face_state* pf, uint64_t pnf, uint64_t generation, const int32_t* cells, uint64_t nc,
                    int64_t* old, fl_block_state* ob, fl_cell_state* oc, fl_face_state* of);
 
+// Where a sorted record list came from a bit set over a cell box: the bits, the scan of their words'
+// popcounts and the box (rows of row_words words), so that a key's position is one word and one scan
+// entry. Empty (null words) for lists of a caller's, which are searched.
+struct KeyIndex {
+  const uint64_t* words = nullptr;
+  const uint64_t* scan = nullptr;
+  int32_t lo[3] = {0, 0, 0}, dim[3] = {0, 0, 0};
+  int32_t row_words = 0;
+};
+// The sorted block list with, for the context's own grid, its dense ordinal table (null: searched).
+struct BlockIndex {
+  const fl_int3* blocks = nullptr;
+  uint64_t nb = 0;
+  const int32_t* lut = nullptr;
+  Box box;
+};
+
 // Typed pressure links of a frozen view (links.hip): device copies of the view and the fields.
 struct LinkDevice {
   const fl_int3* blocks;
@@ -278,6 +295,12 @@ struct LinkDevice {
   uint64_t nair;
   const fl_internal_interface* interfaces;
   uint64_t ninterfaces;
+  // The substep's indices: blocks, centre samples, the frozen cells through their candidates (keep and its
+  // scan), and the frozen faces' slot bitmap. Empty for a caller's view.
+  BlockIndex block_index;
+  KeyIndex centre_index, candidate_index;
+  const uint64_t *keep, *keep_scan;
+  const unsigned long long* face_words;
 };
 // Frozen-geometry device arrays: inputs, per-candidate staging, the face-slot bitmap and the outputs.
 struct FreezeDevice {
@@ -307,7 +330,7 @@ struct FreezeDevice {
   uint64_t* counts;       // 5: kept cells, unique faces, curvature needed, cells listed from the front / back of work
   double* phi;            // 9 * ncand: corner and centre samples of the cut cells
   uint64_t* work;         // ncand: the cut cells
-  double* uncut_volume;   // 2: the uncut cell's volume, plane mode then sampled mode
+  double* uncut_volume;   // 3: the uncut cell's volume (plane mode, sampled mode) and its box measure
   // Sampled solid (sampled != 0): corner samples, dense face normal velocities (count 0: none), and the
   // eight solid corner distances of each listed cell.
   int sampled;
@@ -316,6 +339,9 @@ struct FreezeDevice {
   const double* face_velocities;
   uint64_t nface_velocities;
   double* solid_phi;  // 8 * ncand
+  // The substep's indices of blocks, centre, corner and solid samples (empty for a caller's lists).
+  BlockIndex block_index;
+  KeyIndex centre_index, corner_index, solid_index;
 };
 // Phases 0-2 (sample and candidate checks, kCell, compaction, unique face slots).
 int freeze_cells_device(fl_ctx* ctx, const FreezeDevice& d);
@@ -338,6 +364,7 @@ struct FieldSamples {
   fl_center_distance* corners;
   uint64_t corner_count;
   fl_int3 cell_box_lo, cell_box_hi;  // a box holding every sample
+  KeyIndex cell_index, centre_index, corner_index;
 };
 int sample_particle_field(fl_ctx* ctx, double radius, uint64_t max_candidates, FieldSamples* out);
 void release_field(fl_ctx* ctx);

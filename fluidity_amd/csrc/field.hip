@@ -539,6 +539,20 @@ int sample_particle_field(fl_ctx* ctx, double radius, uint64_t max_candidates, F
   out->centre_count = ncen;
   out->corners = B.corners;
   out->corner_count = ncor;
+  const auto index = [&](const uint64_t* words, int q) {
+    KeyIndex k;
+    k.words = words;
+    k.scan = B.scans + q * nw;
+    for (int a = 0; a < 3; ++a) {
+      k.lo[a] = box.lo[a];
+      k.dim[a] = box.dim[a];
+    }
+    k.row_words = box.row_words;
+    return k;
+  };
+  out->cell_index = index(B.cand, 0);
+  out->centre_index = index(B.centre, 1);
+  out->corner_index = index(B.corner, 2);
   out->cell_box_lo = fl_int3{box.lo[0], box.lo[1], box.lo[2]};
   out->cell_box_hi = fl_int3{box.lo[0] + box.dim[0] - 1, box.lo[1] + box.dim[1] - 1, box.lo[2] + box.dim[2] - 1};
   return FL_OK;

@@ -729,8 +729,8 @@ __device__ int sampled_face_weights(double width, const double (&solid)[4], cons
   return kOk;
 }
 
-__device__ inline double lookup(const fl_center_distance* s, uint64_t n, fl_int3 k, bool& found) {
-  const uint64_t i = find_sorted(s, n, k, [](const fl_center_distance& x) { return x.cell_index; });
+__device__ inline double lookup(const KeyIndex& index, const fl_center_distance* s, uint64_t n, fl_int3 k, bool& found) {
+  const uint64_t i = find_key(index, s, n, k, [](const fl_center_distance& x) { return x.cell_index; });
   found = i != n;
   return found ? s[i].signed_distance : 0.0;
 }
@@ -750,9 +750,10 @@ __global__ void k_check_solids(const fl_solid_corner* s, uint64_t n, uint64_t fi
     fail(err, 1, first + i, kInvalidArgument);
 }
 
-__device__ inline const fl_solid_corner* lookup_solid(const fl_solid_corner* s, uint64_t n, fl_int3 k) {
-  const uint64_t i = find_sorted(s, n, k, [](const fl_solid_corner& x) { return x.corner_index; });
-  return i != n ? s + i : nullptr;
+__device__ inline const fl_solid_corner* lookup_solid(const FreezeDevice& d, fl_int3 k) {
+  const uint64_t i =
+      find_key(d.solid_index, d.solids, d.nsolids, k, [](const fl_solid_corner& x) { return x.corner_index; });
+  return i != d.nsolids ? d.solids + i : nullptr;
 }
 
 // Tetrahedron t's part of the liquid volume on each side of the obstacle of a cell with corner distances
@@ -813,12 +814,14 @@ __device__ void consume_cell(const FreezeDevice& d, uint64_t i, fl_int3 c, doubl
   const double vol = min_std(d.full_volume, unclamped);
   if (!normal_or_zero(vol)) return fail(err, 2, i, kOutOfRange);
   if (center >= 0 || vol == 0) return;
+#pragma unroll
   for (int a = 0; a < 3; ++a)
+#pragma unroll
     for (int side = 0; side < 2; ++side) {
-      fl_int3 l;
-      if (!offset(c, a, side, l)) return fail(err, 2, i, kOutOfRange);
+      if (side && (a == 0 ? c.x : (a == 1 ? c.y : c.z)) == kI32Max) return fail(err, 2, i, kOutOfRange);
+      const fl_int3 l{c.x + (a == 0 ? side : 0), c.y + (a == 1 ? side : 0), c.z + (a == 2 ? side : 0)};
       uint64_t slot = 0;
-      if (int code = sorted_face_slot(d.blocks, d.nb, a, l, slot)) return fail(err, 2, i, code);
+      if (int code = indexed_face_slot(d.block_index, a, l, slot)) return fail(err, 2, i, code);
       d.slots[6 * i + 2 * a + side] = slot;
     }
   fl_frozen_cell r{};
@@ -841,6 +844,7 @@ __global__ void k_uncut_volume(FreezeDevice d) {
   if (t < 6) tet_volumes<false>(phi, t, P, d.h, nullptr, low, high);
   high = sum_tets(high, 0);
   if (t == 0) d.uncut_volume[0] = high;
+  if (t == 0) d.uncut_volume[2] = tank_box_measure(TankBounds{{0, 0, 0}, {1, 1, 1}}, d.h, -1);
   if (d.sampled) {  // the sampled measure of a cell that no plane cuts: its clips return their inputs
     const double solid[8] = {1, 1, 1, 1, 1, 1, 1, 1};
     double wet = 0;
@@ -877,13 +881,39 @@ __device__ inline bool clear_of(const Plane& plane, int side) {
   return true;
 }
 
+// Places for the lanes that are here together, from one atomic on the counter.
+__device__ inline uint64_t take_places(uint64_t* counter) {
+  const uint64_t lanes = __ballot(1);
+  const int lane = static_cast<int>(threadIdx.x & 63), leader = __ffsll(static_cast<long long>(lanes)) - 1;
+  unsigned long long w = 0;
+  if (lane == leader)
+    w = atomicAdd(reinterpret_cast<unsigned long long*>(counter), static_cast<unsigned long long>(__popcll(lanes)));
+  return __shfl(w, leader) + __popcll(lanes & ((uint64_t(1) << lane) - 1));
+}
+
 // Lists a cut cell with its samples: cells that only the liquid surface cuts from the front of the work
 // list, cells that obstacle planes or the sampled solid may cut too from its back.
 __device__ inline void list_cut(const FreezeDevice& d, uint64_t i, const double (&phi)[8], double center, bool planes) {
+#pragma unroll
   for (int k = 0; k < 8; ++k) d.phi[9 * i + k] = phi[k];
   d.phi[9 * i + 8] = center;
-  const unsigned long long w = atomicAdd(reinterpret_cast<unsigned long long*>(d.counts + (planes ? 4 : 3)), 1ull);
-  d.work[planes ? d.ncand - 1 - w : w] = i;
+  if (planes) d.work[d.ncand - 1 - take_places(d.counts + 4)] = i;
+  else d.work[take_places(d.counts + 3)] = i;
+}
+
+// The bounded sums of a cell's six walls and extents, and one 64-bit atomic per listed lane, were most of the
+// staging kernel: 1.22 ms for 0.7M candidates, now 0.21 ms with this test and the wave's one atomic.
+// Whether the tank's walls clearly miss the element at c, by far more than the rounding of the bounded
+// sums that locate them: its walls are then the unit cell's faces and its world extent is resolved.
+__device__ inline bool clear_of_walls(const FreezeDevice& d, fl_int3 c) {
+  const fl_tank& t = d.obstacle.tank;
+  const auto clear = [&](double origin, int32_t index, double low_wall, double high_wall) {
+    const double low = origin + d.h * index, high = origin + d.h * (double(index) + 1);
+    const double margin = 1e-6 * d.h;
+    return (fabs(origin) + fabs(low) + fabs(high)) * 1e-9 < margin && low_wall < low - margin && high_wall > high + margin;
+  };
+  return clear(d.origin.x, c.x, t.start_low_x, t.high_x) && clear(d.origin.y, c.y, t.floor_y, __builtin_inf()) &&
+         clear(d.origin.z, c.z, t.low_z, t.high_z);
 }
 
 // One lane per candidate: order check and sample lookups, then the kCell query for the cells it settles
@@ -898,18 +928,19 @@ __global__ void k_freeze_stage(FreezeDevice d, uint64_t* err) {
   const fl_int3 c = d.candidates[i];
   if (i > 0 && !key_less(d.candidates[i - 1], c)) return fail(err, 2, i, kInvalidArgument);
   bool found = false;
-  const double center = lookup(d.centers, d.ncenters, c, found);
+  const double center = lookup(d.centre_index, d.centers, d.ncenters, c, found);
   if (!found) return fail(err, 2, i, kFailedPrecondition);
   double phi[8];
   bool any_negative = false, all_negative = true;
+#pragma unroll
   for (int k = 0; k < 8; ++k) {
-    fl_int3 q = c;
-    for (int a = 0; a < 3; ++a)
-      if (!offset(q, a, (k >> a) & 1, q)) return fail(err, 2, i, kOutOfRange);
-    phi[k] = lookup(d.corners, d.ncorners, q, found);
+    const int ox = k & 1, oy = (k >> 1) & 1, oz = k >> 2;
+    if ((ox && c.x == kI32Max) || (oy && c.y == kI32Max) || (oz && c.z == kI32Max)) return fail(err, 2, i, kOutOfRange);
+    const fl_int3 q{c.x + ox, c.y + oy, c.z + oz};
+    phi[k] = lookup(d.corner_index, d.corners, d.ncorners, q, found);
     if (!found) return fail(err, 2, i, kFailedPrecondition);
     if (d.sampled) {
-      const fl_solid_corner* solid = lookup_solid(d.solids, d.nsolids, q);
+      const fl_solid_corner* solid = lookup_solid(d, q);
       if (!solid) return fail(err, 2, i, kFailedPrecondition);
       d.solid_phi[8 * i + k] = solid->signed_distance;
     }
@@ -943,9 +974,14 @@ __global__ void k_freeze_stage(FreezeDevice d, uint64_t* err) {
     }
     return list_cut(d, i, phi, center, !clear);
   }
-  Planes P;
-  if (int code = local_planes(d, c, P)) return fail(err, 2, i, code);
   if (d.obstacle.kind == FL_OBSTACLE_TANK) {  // the tank cell's box, or the liquid inside it
+    if (clear_of_walls(d, c)) {  // the whole box, whose measure depends on h alone
+      const double box = d.uncut_volume[2];
+      if (!normal_or_zero(box)) return fail(err, 2, i, kOutOfRange);
+      if (box == 0 || !any_negative) return consume_cell(d, i, c, center, 0.0, 0.0, err);
+      if (all_negative) return consume_cell(d, i, c, center, 0.0, box, err);
+      return list_cut(d, i, phi, center, false);
+    }
     if (!tank_cell_resolved(d, c)) return fail(err, 2, i, kOutOfRange);
     TankBounds tb;
     if (int code = local_tank_bounds(d, c, -1, tb)) return fail(err, 2, i, code);
@@ -957,6 +993,8 @@ __global__ void k_freeze_stage(FreezeDevice d, uint64_t* err) {
     for (int a = 0; a < 3; ++a) walled = walled || tb.low[a] > 0 || tb.high[a] < 1;
     return list_cut(d, i, phi, center, walled);
   }
+  Planes P;
+  if (int code = local_planes(d, c, P)) return fail(err, 2, i, code);
   if (!any_negative) return consume_cell(d, i, c, center, 0.0, 0.0, err);
   if (all_negative) {
     const bool high_whole = !P.present || all_kept(Plane{scale(P.normal, -1), -P.high, false});
@@ -973,12 +1011,14 @@ __global__ void k_freeze_stage(FreezeDevice d, uint64_t* err) {
 // polygons in private memory (dependent FP64 and scratch accesses), so the chain is what is cut: one
 // tetrahedron per lane instead of six in turn, and a quarter of the private memory where no obstacle
 // plane joins the liquid surface. Per substep of 16^3 / 150^3 tank scenes (7,680 / 4.5M particles) 1.45 /
-// 4.27 ms with one lane per cell, now 0.05 + 0.22 / 0.46 + 1.19 ms (surface-only cells + wall cells); of
+// 4.27 ms with one lane per cell, now 0.04 + 0.19 / 0.41 + 0.93 ms (surface-only cells + wall cells); of
 // the stirred 128^3 scene with its face areas 2.84 ms, now 1.45 ms.
 constexpr int kCutCells = 10;
 constexpr uint64_t kCutWaves = 256 * 4 * 4;  // four waves on every SIMD
-template <bool kPlanes>
+enum CutMode { kSurfaceCut, kPlaneCut, kSolidCut };
+template <CutMode kMode>
 __global__ void __launch_bounds__(64) k_freeze_cut(FreezeDevice d, uint64_t* err) {
+  constexpr bool kPlanes = kMode != kSurfaceCut;
   const uint64_t listed = d.counts[kPlanes ? 4 : 3];
   const int group = static_cast<int>(threadIdx.x) / 6, t = static_cast<int>(threadIdx.x) % 6, base = 6 * group;
   const bool lane = group < kCutCells;
@@ -993,27 +1033,26 @@ __global__ void __launch_bounds__(64) k_freeze_cut(FreezeDevice d, uint64_t* err
     for (int k = 0; k < 8; ++k) phi[k] = d.phi[9 * i + k];
     double low = 0, high = 0;
     int code = kOk;
-    if constexpr (kPlanes) {
+    if constexpr (kMode == kSolidCut) {  // ComputeSampledSolidGeometry for a cell: the wet volume as the high side's
       Planes P;
-      if (d.sampled) {  // ComputeSampledSolidGeometry for a cell: the wet volume as the high side's
-        code = local_planes(d, c, P);
-        if (code == kOk && d.obstacle.kind != FL_OBSTACLE_ABSENT && d.obstacle.kind != FL_OBSTACLE_HALFSPACE)
-          code = kInvalidArgument;
-        double solid[8];
-        for (int k = 0; k < 8; ++k) solid[k] = d.solid_phi[8 * i + k];
-        const Plane analytic{scale(P.normal, -1), -P.high, false};
-        const int measured =
-            measure_sampled_cell(d.h, phi, solid, P.present ? &analytic : nullptr, high, d.sampled, use ? t : 6, from);
-        if (code == kOk) code = measured;
-      } else {
-        (void)local_planes(d, c, P);  // succeeded in k_freeze_stage
-        TankBounds tb;
-        const bool tank = d.obstacle.kind == FL_OBSTACLE_TANK;
-        if (tank) (void)local_tank_bounds(d, c, -1, tb);  // succeeded in k_freeze_stage
-        if (use) tet_volumes<true>(phi, t, P, d.h, tank ? &tb : nullptr, low, high);
-        low = sum_tets(low, from);
-        high = sum_tets(high, from);
-      }
+      code = local_planes(d, c, P);
+      if (code == kOk && d.obstacle.kind != FL_OBSTACLE_ABSENT && d.obstacle.kind != FL_OBSTACLE_HALFSPACE)
+        code = kInvalidArgument;
+      double solid[8];
+      for (int k = 0; k < 8; ++k) solid[k] = d.solid_phi[8 * i + k];
+      const Plane analytic{scale(P.normal, -1), -P.high, false};
+      const int measured =
+          measure_sampled_cell(d.h, phi, solid, P.present ? &analytic : nullptr, high, d.sampled, use ? t : 6, from);
+      if (code == kOk) code = measured;
+    } else if constexpr (kMode == kPlaneCut) {
+      Planes P;
+      (void)local_planes(d, c, P);  // succeeded in k_freeze_stage
+      TankBounds tb;
+      const bool tank = d.obstacle.kind == FL_OBSTACLE_TANK;
+      if (tank) (void)local_tank_bounds(d, c, -1, tb);  // succeeded in k_freeze_stage
+      if (use) tet_volumes<true>(phi, t, P, d.h, tank ? &tb : nullptr, low, high);
+      low = sum_tets(low, from);
+      high = sum_tets(high, from);
     } else {
       if (use) tet_volumes<false>(phi, t, Planes{}, d.h, nullptr, low, high);
       high = sum_tets(high, from);
@@ -1111,7 +1150,7 @@ __device__ int sampled_face(const FreezeDevice& d, fl_int3 l, int axis, uint64_t
     fl_int3 q = l;
     for (int a = 0; a < 3; ++a)
       if (!offset(q, a, (k >> a) & 1, q)) return kOutOfRange;
-    const fl_solid_corner* sample = lookup_solid(d.solids, d.nsolids, q);
+    const fl_solid_corner* sample = lookup_solid(d, q);
     if (!sample) return kFailedPrecondition;
     solid[k] = sample->signed_distance;
     const double wv[3] = {sample->wall_velocity.x, sample->wall_velocity.y, sample->wall_velocity.z};
@@ -1263,7 +1302,7 @@ __global__ void k_curvature_needs(FreezeDevice d, uint64_t nc, uint64_t nf, uint
   const bool has_head = hc != nc, has_tail = tc != nc;
   if (has_head && has_tail) return;
   bool found = false;
-  const double air = lookup(d.centers, d.ncenters, has_head ? tail : head, found);
+  const double air = lookup(d.centre_index, d.centers, d.ncenters, has_head ? tail : head, found);
   if (!found) return fail(err, 4, j, kFailedPrecondition);
   if (air >= 0) {
     d.needs[has_head ? hc : tc] = 1;
@@ -1291,7 +1330,7 @@ __global__ void k_curvature(FreezeDevice d, uint64_t nc, uint64_t* err) {
         for (int a = 0; a < 3; ++a)
           if (!offset(q, a, o[a], q)) return fail(err, 5, i, kOutOfRange);
         bool found = false;
-        s[(z + 1) * 9 + (y + 1) * 3 + x + 1] = lookup(d.centers, d.ncenters, q, found);
+        s[(z + 1) * 9 + (y + 1) * 3 + x + 1] = lookup(d.centre_index, d.centers, d.ncenters, q, found);
         if (!found) return fail(err, 5, i, kFailedPrecondition);
       }
   const double h = d.h;
@@ -1338,8 +1377,9 @@ int freeze_cells_device(fl_ctx* ctx, const FreezeDevice& d) {
     k_freeze_stage<<<grid_for(d.ncand), kThreads, 0, s>>>(d, ctx->err);
     // Grids that fill the chip once; the lists' lengths stay on the device.
     const unsigned waves = static_cast<unsigned>(std::min<uint64_t>((d.ncand + kCutCells - 1) / kCutCells, kCutWaves));
-    k_freeze_cut<false><<<waves, 64, 0, s>>>(d, ctx->err);
-    if (d.sampled || d.obstacle.kind != FL_OBSTACLE_ABSENT) k_freeze_cut<true><<<waves, 64, 0, s>>>(d, ctx->err);
+    k_freeze_cut<kSurfaceCut><<<waves, 64, 0, s>>>(d, ctx->err);
+    if (d.sampled) k_freeze_cut<kSolidCut><<<waves, 64, 0, s>>>(d, ctx->err);
+    else if (d.obstacle.kind != FL_OBSTACLE_ABSENT) k_freeze_cut<kPlaneCut><<<waves, 64, 0, s>>>(d, ctx->err);
     FL_TRY(exclusive_scan_u64(ctx, d.keep, d.keep_scan, d.ncand));
     k_compact_cells<<<grid_for(d.ncand), kThreads, 0, s>>>(d);
   }

@@ -26,14 +26,24 @@ struct View {
   const fl_frozen_face* faces;
   uint64_t nfaces;
   double h, step, density, sigma;
+  BlockIndex block_index;
+  KeyIndex centre_index, candidate_index;
+  const uint64_t *keep, *keep_scan;
+  const unsigned long long* face_words;
 };
 
+// Position of the frozen cell at k, or ncells: through its candidate where the cells came from one.
 __device__ inline uint64_t find_cell(const View& v, fl_int3 k) {
+  if (v.candidate_index.words) {
+    const uint64_t none = ~uint64_t(0);
+    const uint64_t i = find_key(v.candidate_index, v.cells, none, k, [](const fl_frozen_cell& c) { return c.cell_index; });
+    return i != none && v.keep[i] ? v.keep_scan[i] : v.ncells;
+  }
   return find_sorted(v.cells, v.ncells, k, [](const fl_frozen_cell& c) { return c.cell_index; });
 }
 
 __device__ inline int face_slot(const View& v, int axis, fl_int3 l, uint64_t& slot) {
-  return sorted_face_slot(v.blocks, v.nb, axis, l, slot);
+  return indexed_face_slot(v.block_index, axis, l, slot);
 }
 
 __global__ void k_check_centers(View v, uint64_t* err) {
@@ -96,6 +106,10 @@ __global__ void k_check_incident(View v, uint64_t* err) {
     fail(err, 3, t, code);
     return;
   }
+  if (v.face_words) {
+    if (!((v.face_words[slot / 64] >> (slot % 64)) & 1)) fail(err, 3, t, kFailedPrecondition);
+    return;
+  }
   uint64_t lo = 0, hi = v.nfaces;
   while (lo < hi) {
     const uint64_t mid = lo + (hi - lo) / 2;
@@ -136,7 +150,7 @@ __global__ void k_check_air(View v, Fields F, uint64_t* err) {
     return;
   }
   const uint64_t s =
-      find_sorted(v.centers, v.ncenters, a.cell_index, [](const fl_center_distance& c) { return c.cell_index; });
+      find_key(v.centre_index, v.centers, v.ncenters, a.cell_index, [](const fl_center_distance& c) { return c.cell_index; });
   if (s == v.ncenters) fail(err, 5, i, kFailedPrecondition);
   else if (v.centers[s].signed_distance < 0.0 || find_cell(v, a.cell_index) != v.ncells)
     fail(err, 5, i, kInvalidArgument);
@@ -301,7 +315,7 @@ __global__ void k_link_faces(View v, Fields F, fl_pressure_face* out, unsigned l
   } else if (face.open_area > 0) {
     const fl_int3 air_cell = has_head ? tail : head;
     const uint64_t s =
-        find_sorted(v.centers, v.ncenters, air_cell, [](const fl_center_distance& c) { return c.cell_index; });
+        find_key(v.centre_index, v.centers, v.ncenters, air_cell, [](const fl_center_distance& c) { return c.cell_index; });
     if (s == v.ncenters || v.centers[s].signed_distance < 0) {
       fail(err, 7, i, kFailedPrecondition);
       return;
@@ -337,7 +351,8 @@ int build_links_device(fl_ctx* ctx, const LinkDevice& d, fl_pressure_cell* out_c
                        uint64_t* d_lower, bool validate_only) {
   hipStream_t s = ctx->stream;
   const View v{d.blocks, d.nb, d.centers, d.ncenters, d.cells, d.ncells, d.faces, d.nfaces,
-               d.h, d.step, d.density, d.sigma};
+               d.h, d.step, d.density, d.sigma, d.block_index, d.centre_index, d.candidate_index, d.keep, d.keep_scan,
+               d.face_words};
   if (validate_only) {
     const double full_area = d.h * d.h, full_volume = full_area * d.h;
     if (v.ncenters) k_check_centers<<<grid_for(v.ncenters), kThreads, 0, s>>>(v, ctx->err);

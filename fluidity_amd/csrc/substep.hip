@@ -361,7 +361,7 @@ int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep) {
   FL_TRY(grow_to(&B.counts, &B.cap[13], 5));
   FL_TRY(grow_to(&B.phi, &B.cap[14], 9 * ncand));
   FL_TRY(grow_to(&B.work, &B.cap[15], ncand));
-  FL_TRY(grow_to(&B.uncut, &B.cap[16], 2));
+  FL_TRY(grow_to(&B.uncut, &B.cap[16], 3));
   const double full_area = h * h, full_volume = full_area * h;
   const FreezeDevice fd{reinterpret_cast<const fl_int3*>(ctx->blocks),
                         nb,
@@ -398,6 +398,10 @@ int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep) {
                         0,
                         nullptr};
   FreezeDevice fd_run = fd;
+  const BlockIndex block_index{reinterpret_cast<const fl_int3*>(ctx->blocks), nb, ctx->lut, ctx->block_box};
+  fd_run.block_index = block_index;
+  fd_run.centre_index = F.centre_index;
+  fd_run.corner_index = F.corner_index;
   if (o.solid.parts) {
     FL_TRY(grow_to(&B.solids, &B.cap[24], F.corner_count));
     FL_TRY(grow_to(&B.solid_phi, &B.cap[25], 8 * ncand));
@@ -420,6 +424,7 @@ int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep) {
     fd_run.solids = B.solids;
     fd_run.nsolids = F.corner_count;
     fd_run.solid_phi = B.solid_phi;
+    fd_run.solid_index = F.corner_index;  // one solid sample per corner sample, in its order
   }
   auto read_counts = [&]() -> int {
     FL_HIP(hipMemcpyAsync(ctx->host_words, B.counts, 3 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
@@ -462,7 +467,8 @@ int substep(fl_ctx* ctx, const fl_substep_options& o, fl_substep_report& rep) {
   {
     const LinkDevice ld{reinterpret_cast<const fl_int3*>(ctx->blocks), nb, F.centres, F.centre_count, B.cells, nc,
                         B.faces, nf, h, dt, o.liquid_density, o.surface_tension, B.fields, B.predicted,
-                        o.ambient_pressure, nullptr, 0, nullptr, 0, nullptr, 0};
+                        o.ambient_pressure, nullptr, 0, nullptr, 0, nullptr, 0, block_index, F.centre_index,
+                        F.cell_index, B.keep, B.keep + ncand, B.words};
     FL_TRY(reset_error(ctx));
     STAGE(5, build_links_device(ctx, ld, nullptr, nullptr, nullptr, true));
     STAGE(5, error_code(ctx));

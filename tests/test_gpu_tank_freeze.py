@@ -86,3 +86,15 @@ def test_pool_in_tank(ctx):
     assert s_want == O.OK and s_got == s_want and gl == wl
     same(gc.view(O.PRESSURE_CELL), wc)
     same(gf.view(O.PRESSURE_FACE), wf)
+
+
+@pytest.mark.parametrize("eps", [0.0, 1e-17, 1e-9, 1e-7, 3e-6])
+def test_walls_beside_the_lattice(ctx, eps):
+    """Tank walls on and just beside lattice planes: the cells that they clearly miss skip the bounded sums, the
+    ones they may touch do not, with the oracle's bits and status."""
+    n = 20
+    for side in (-1.0, 1.0):
+        p = pool_in_tank(n)
+        e = side * eps / n
+        p.obstacle = T.tank(2.0 / n + e, 18.0 / n - e, 1.0 / n + e, 2.0 / n - e, 18.0 / n + e, 0.37)
+        check(ctx, p)
