@@ -113,6 +113,29 @@ def test_device_built_projection_equals_host_built(ctx):
     assert np.max(np.abs(p - want["pressures"])) <= 1e-5 * np.max(np.abs(want["pressures"]))
 
 
+@pytest.mark.parametrize("share", [0.25, 0.45, 0.7, 1.0])
+@pytest.mark.parametrize("n", [9, 12])
+def test_device_built_components(ctx, n, share):
+    """Liquids of many components, within and across the 4^3 blocks (cells drawn at random), and a sealed
+    full box (no anchor: the host's gauge): the device-built system equals the host-built one bit for bit."""
+    rng = np.random.default_rng(int(100 * share) + n)
+    liquid = rng.random((n, n, n)) < share
+    sc = scenes.Scene("drops", n, 0, liquid, np.zeros((0, 3)), np.zeros((0, 3)), np.zeros((0, 3, 3)), 1.0)
+    b = np.arange(-1, n // 4 + 2)
+    z, y, x = np.meshgrid(b, b, b, indexing="ij")
+    blocks = np.zeros(x.size, R.INT3)
+    blocks["x"], blocks["y"], blocks["z"] = x.ravel(), y.ravel(), z.ravel()
+    faces = sc.pressure_faces(blocks, rng.normal(0.0, 1.0, 192 * len(blocks)))
+    geom = O.geometry((0.0, 0.0, 0.0), sc.h)
+    opts = H.pressure_options(relative_target=1e-8, levels=2, sweeps=2)
+    s, host = ctx.project(geom, blocks, 1e-3, sc.pressure_cells(), faces, opts)
+    s2, p, u, diag = ctx.project_device_built(geom, blocks, 1e-3, sc.pressure_cells(), faces, opts)
+    assert s == s2 == H.OK
+    assert diag["iteration_count"] == host["diagnostics"]["iteration_count"]
+    assert np.array_equal(p.view(np.uint64), host["pressures"].view(np.uint64))
+    assert np.array_equal(u.view(np.uint64), host["velocities"].view(np.uint64))
+
+
 def test_substep_chain_matches_oracle(ctx):
     sc = scenes.dam_break(16, seed=3)
     geom = O.geometry((0.0, 0.0, 0.0), sc.h)
