@@ -19,6 +19,7 @@
 #include <cstring>
 #include <limits>
 #include <numeric>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -696,7 +697,6 @@ __global__ void k_diag(uint64_t n, const int32_t* nbr, const float* k, const flo
 
 // ------------------------------------------------------------------ V-cycle kernels (FP32)
 
-// Per-cell V-cycle operations, shared by the grid-wide kernels and the single-workgroup tail cycle.
 template <class KT>
 struct LevelViewT {
   uint64_t n;             // cells (64 per block)
@@ -740,36 +740,6 @@ __device__ inline void smooth_cell(const LevelViewT<KT>& L, uint64_t t, int colo
     for (int dir = 0; dir < 6; ++dir) s += kk[dir] * xx[dir];
   }
   L.x[i] = d == 0.f ? 0.f : s / d;
-}
-
-// Coarse right-hand side of coarse cell ci: the sum of the fine residuals b - A x of its 2x2x2
-// children. Pre-smoothing ends with a black half sweep, which leaves every black (odd) cell's
-// equation satisfied, so only the four red children carry a residual.
-template <class KT>
-__device__ inline float restrict_residual(const LevelViewT<KT>& F, const int32_t* child, uint64_t ci) {
-  const uint64_t blk = ci >> 6;
-  const int l = cnat(static_cast<int>(ci & 63));
-  const int cx = l & 3, cy = (l >> 2) & 3, cz = l >> 4;
-  float sum = 0.f;
-  for (int o = 0; o < 8; ++o) {
-    const int ox = o & 1, oy = (o >> 1) & 1, oz = o >> 2;
-    if (((ox + oy + oz) & 1) != 0) continue;  // fine parity = own parity (2c is even): odd octants are black
-    const int fx = 2 * cx + ox, fy = 2 * cy + oy, fz = 2 * cz + oz;
-    const int32_t fb = child[8 * blk + ((fz >> 2) * 2 + (fy >> 2)) * 2 + (fx >> 2)];
-    if (fb < 0) continue;
-    const int lx = fx & 3, ly = fy & 3, lz = fz & 3;
-    const uint64_t fi = uint64_t(fb) * 64 + cslot(lz * 16 + ly * 4 + lx);
-    if (F.diag[fi] == 0.f) continue;
-    const float xi = F.x[fi];
-    float a = F.anchor[fi] * xi;
-    for (int dir = 0; dir < 6; ++dir) {
-      const int64_t j = neighbour(F.nbr, uint64_t(fb), lx, ly, lz, dir);
-      if (j < 0) continue;
-      a += face_kt(F.k, F.n, static_cast<int64_t>(fi), j, dir) * (xi - F.x[j]);
-    }
-    sum += F.b[fi] - a;
-  }
-  return sum;
 }
 
 // x_fine += x_coarse(parent).
@@ -962,55 +932,257 @@ __global__ void k_restrict_all(const float* r, LevelViewT<KT> C) {
   const_cast<float*>(C.b)[i] = sum;
 }
 
+// ---- The small levels, in one workgroup with every value in LDS ----
+// The levels from the first of at most kTailBlocks blocks down to the coarsest are a few thousand cells:
+// the work is nothing, and what counts is the chain of dependent steps (a half sweep waits for the one
+// before it), so what counts is the latency of one step. The workgroup copies the levels' right-hand
+// sides and coefficients into LDS in one go and then works there: one lane holds the coefficients and
+// LDS positions of one red and one black cell (of two of each above 32 blocks) in registers for all the
+// sweeps of a level visit, so that a half sweep is six LDS reads, the sum and the division. Levels of at
+// most two blocks are one wave and need no barrier. With the values in global memory a half sweep waited
+// for the block table, then the coefficients and neighbours: 29.4 us instead of TAIL_MEASURED for three levels
+// from 24 blocks on (two sweeps, two symmetric sweeps on the coarsest level).
+// The bounds are LDS: 24 B per cell of all of these levels, and the directions of the first one (the anchors,
+// which the sweeps do not use, stay in global memory). A level that does not fit costs eleven launches of
+// 4 us per cycle.
 constexpr int kMaxTail = 16;
-constexpr uint64_t kTailBlocks = 32;  // levels with at most this many blocks run in the tail cycle
+constexpr uint64_t kTailBlocks = 64;  // of the first of these levels
+constexpr int kTailStore = 92;        // of all of these levels together
+constexpr int kTailLanes = 1024;
 template <class KT>
 struct TailCycle {
   int count, nu, coarse_sweeps;
+  int first[kMaxTail + 1];  // first block of each level in the workgroup's arrays
   LevelViewT<KT> lv[kMaxTail];
 };
 
-// The V-cycle below and including the first small level, in one workgroup: pre-smoothing and
-// residual restriction down to the coarsest level, symmetric sweeps there from zero, then
-// prolongation and post-smoothing back up. Barriers separate the dependent steps; every wave of the
-// workgroup shares the CU's vector cache, so each step sees the previous one's stores.
+struct TailStore {
+  float x[kTailStore * 64 + 1];  // one more: the zero that stands for a missing neighbour
+  float b[kTailStore * 64], d[kTailStore * 64], k[3][kTailStore * 64];
+  // Residuals of a level's red cells during the cycle; outside it, a search direction and the zero of a
+  // missing neighbour.
+  float r[kTailBlocks * 64 + 1];
+  int16_t nbr[kTailStore][6], child[kTailStore][8], parent[kTailStore][2];
+};
+
+// The two cells (slot s of the red half and of the black half of a block) of a lane.
+struct TailPair {
+  bool live;
+  int i[2];
+  int16_t j[2][6];
+  float k[2][6], d[2], b[2];
+};
+
 template <class KT>
-__global__ __launch_bounds__(1024) void k_tail_vcycle(TailCycle<KT> T) {
-  const uint64_t tid = threadIdx.x, nt = blockDim.x;
-  auto sync = [] {
-    __threadfence_block();
-    __syncthreads();
+__device__ inline void tail_load(const TailCycle<KT>& T, TailStore& S) {
+  const int tid = threadIdx.x, nt = blockDim.x;
+  for (int q = 0; q < T.count; ++q) {
+    const LevelViewT<KT>& L = T.lv[q];
+    const int o = T.first[q], nb = T.first[q + 1] - o;
+    for (int i = tid; i < nb * 64; i += nt) {
+      const int w = o * 64 + i;
+      if (q == 0) S.b[w] = L.b[i];
+      S.d[w] = L.diag[i];
+      for (int axis = 0; axis < 3; ++axis) S.k[axis][w] = kload(L.k, int64_t(axis) * int64_t(L.n) + i);
+    }
+    for (int i = tid; i < nb * 6; i += nt) {
+      const int32_t v = L.nbr[i];
+      S.nbr[o + i / 6][i % 6] = static_cast<int16_t>(v < 0 ? -1 : v + o);
+    }
+    if (q > 0)
+      for (int i = tid; i < nb * 8; i += nt) {
+        const int32_t v = L.child[i];
+        S.child[o + i / 8][i % 8] = static_cast<int16_t>(v < 0 ? -1 : v + T.first[q - 1]);
+      }
+    if (q + 1 < T.count)
+      for (int i = tid; i < nb * 2; i += nt) {
+        const int32_t v = L.parent[i];
+        S.parent[o + i / 2][i % 2] = static_cast<int16_t>((i & 1) || v < 0 ? v : v + T.first[q + 1]);
+      }
+  }
+  if (tid == 0) S.x[kTailStore * 64] = 0.f;
+  __syncthreads();
+}
+
+// A lane's h-th pair of the level of blocks [first, next).
+__device__ inline int tail_block(int h) { return (threadIdx.x >> 5) + h * (kTailLanes / 32); }
+
+__device__ inline TailPair tail_pair(const TailStore& S, int first, int next, int h) {
+  TailPair P;
+  const int blk = first + tail_block(h);
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // positions within the block are formed per visit, not kept over the iterations
+  P.live = blk < next;
+  if (!P.live) return P;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int sl = (c << 5) | (t & 31), l = cnat(sl), i = blk * 64 + sl;
+    const int at[3] = {l & 3, (l >> 2) & 3, l >> 4};
+    P.i[c] = i;
+    P.d[c] = S.d[i];
+    P.b[c] = S.b[i];
+#pragma unroll
+    for (int dir = 0; dir < 6; ++dir) {
+      const int axis = dir >> 1, step = 1 << (2 * axis);
+      const bool outside = at[axis] == ((dir & 1) ? 3 : 0);
+      const int nb = outside ? S.nbr[blk][dir] : blk;
+      const int nl = (dir & 1) ? (outside ? l - 3 * step : l + step) : (outside ? l + 3 * step : l - step);
+      const int j = nb * 64 + cslot(nl);
+      P.j[c][dir] = static_cast<int16_t>(nb < 0 ? kTailStore * 64 : j);
+      P.k[c][dir] = nb < 0 ? 0.f : S.k[axis][(dir & 1) ? j : i];
+    }
+  }
+  return P;
+}
+
+template <int C>
+__device__ inline void tail_smooth(const TailPair& P, TailStore& S, bool first) {
+  if (!P.live) return;
+  float s = P.b[C];
+  if (!first) {
+    float xx[6];
+#pragma unroll
+    for (int dir = 0; dir < 6; ++dir) xx[dir] = S.x[P.j[C][dir]];
+#pragma unroll
+    for (int dir = 0; dir < 6; ++dir) s += P.k[C][dir] * xx[dir];
+  }
+  S.x[P.i[C]] = P.d[C] == 0.f ? 0.f : s / P.d[C];
+}
+
+// The V-cycle of the stored levels from S.b of the first one, into S.x: pre-smoothing and the residual's
+// restriction down to the coarsest level, symmetric sweeps there from zero, then prolongation and
+// post-smoothing back up. Every lane of the workgroup calls it.
+template <class KT, int kPairs>
+__device__ inline void tail_cycle(const TailCycle<KT>& T, TailStore& S) {
+  const int t = threadIdx.x;
+  // A step of a level of one or two blocks belongs to the first wave alone, whose LDS operations are in
+  // order; the other waves wait at the barrier that ends the level's visit.
+  auto step = [](bool solo) {
+    if (solo)
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    else
+      __syncthreads();
+  };
+  TailPair P[kPairs];
+  auto load = [&](int first, int next) {
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) P[h] = tail_pair(S, first, next, h);
+  };
+  auto red = [&](bool first) {
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) tail_smooth<0>(P[h], S, first);
+  };
+  auto black = [&] {
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) tail_smooth<1>(P[h], S, false);
   };
   for (int q = 0; q + 1 < T.count; ++q) {
-    const LevelViewT<KT>& L = T.lv[q];
-    for (int it = 0; it < T.nu; ++it) {
-      for (uint64_t t = tid; t < L.n / 2; t += nt) smooth_cell(L, t, 0, it == 0);
-      sync();
-      for (uint64_t t = tid; t < L.n / 2; t += nt) smooth_cell(L, t, 1, 0);
-      sync();
+    const int first = T.first[q], next = T.first[q + 1];
+    const bool solo = next - first <= 2;
+    if (!solo || t < 64) {
+      load(first, next);
+      float anchor[kPairs];
+#pragma unroll
+      for (int h = 0; h < kPairs; ++h) anchor[h] = P[h].live ? T.lv[q].anchor[P[h].i[0] - 64 * first] : 0.f;
+      for (int it = 0; it < T.nu; ++it) {
+        red(it == 0);
+        step(solo);
+        black();
+        step(solo);
+      }
+      // The closing black half sweep leaves the black cells' equations satisfied: only the four red
+      // children of a coarse cell carry a residual.
+#pragma unroll
+      for (int h = 0; h < kPairs; ++h) {
+        const TailPair& p = P[h];
+        if (!p.live) continue;
+        float r = 0.f;
+        if (p.d[0] != 0.f) {
+          const float xi = S.x[p.i[0]];
+          float a = anchor[h] * xi;
+#pragma unroll
+          for (int dir = 0; dir < 6; ++dir) {
+            const float term = p.k[0][dir] * (xi - S.x[p.j[0][dir]]);
+            if (p.j[0][dir] != kTailStore * 64) a += term;
+          }
+          r = p.b[0] - a;
+        }
+        S.r[32 * tail_block(h) + (t & 31)] = r;
+      }
     }
-    const LevelViewT<KT>& C = T.lv[q + 1];
-    for (uint64_t i = tid; i < C.n; i += nt) const_cast<float*>(C.b)[i] = restrict_residual(L, C.child, i);
-    sync();
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) {
+      const int blk = next + tail_block(h);
+      if (blk >= T.first[q + 2]) continue;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int sl = (c << 5) | (t & 31), l = cnat(sl);
+        const int cx = l & 3, cy = (l >> 2) & 3, cz = l >> 4;
+        float sum = 0.f;
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+          if (((o ^ (o >> 1) ^ (o >> 2)) & 1) != 0) continue;  // fine parity = own parity (2c is even)
+          const int fx = 2 * cx + (o & 1), fy = 2 * cy + ((o >> 1) & 1), fz = 2 * cz + (o >> 2);
+          const int fb = S.child[blk][((fz >> 2) * 2 + (fy >> 2)) * 2 + (fx >> 2)];
+          if (fb >= 0) sum += S.r[(fb - first) * 32 + cslot((fz & 3) * 16 + (fy & 3) * 4 + (fx & 3))];
+        }
+        S.b[blk * 64 + sl] = sum;
+      }
+    }
   }
-  const LevelViewT<KT>& B = T.lv[T.count - 1];
-  for (int pass = 0; pass < 4 * T.coarse_sweeps; ++pass) {
-    const int fwd = pass < 2 * T.coarse_sweeps;
-    const int color = fwd ? (pass & 1) : 1 - (pass & 1);
-    for (uint64_t t = tid; t < B.n / 2; t += nt) smooth_cell(B, t, color, pass == 0);
-    sync();
+  {
+    const int first = T.first[T.count - 1], next = T.first[T.count];
+    const bool solo = next - first <= 2;
+    if (!solo || t < 64) {
+      load(first, next);
+      for (int pass = 0; pass < 4 * T.coarse_sweeps; ++pass) {
+        if ((pass < 2 * T.coarse_sweeps) == ((pass & 1) == 0))
+          red(pass == 0);
+        else
+          black();
+        step(solo);
+      }
+    }
+    __syncthreads();
   }
   for (int q = T.count - 2; q >= 0; --q) {
-    const LevelViewT<KT>& L = T.lv[q];
-    for (uint64_t i = tid; i < L.n; i += nt) prolong_cell(L, T.lv[q + 1].x, i);
-    sync();
-    for (int it = 0; it < T.nu; ++it) {
-      for (uint64_t t = tid; t < L.n / 2; t += nt) smooth_cell(L, t, 1, 0);
-      sync();
-      for (uint64_t t = tid; t < L.n / 2; t += nt) smooth_cell(L, t, 0, 0);
-      sync();
+    const int first = T.first[q], next = T.first[q + 1];
+    const bool solo = next - first <= 2;
+    if (!solo || t < 64) {
+      load(first, next);
+#pragma unroll
+      for (int h = 0; h < kPairs; ++h) {
+        const TailPair& p = P[h];
+        if (!p.live) continue;
+        const int blk = first + tail_block(h);
+        const int pb = S.parent[blk][0], oct = S.parent[blk][1];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int l = cnat((c << 5) | (t & 31));
+          const int px = ((oct & 1) * 4 + (l & 3)) >> 1, py = (((oct >> 1) & 1) * 4 + ((l >> 2) & 3)) >> 1,
+                    pz = ((oct >> 2) * 4 + (l >> 4)) >> 1;
+          if (p.d[c] != 0.f) S.x[p.i[c]] += S.x[pb * 64 + cslot(pz * 16 + py * 4 + px)];
+        }
+      }
+      step(solo);
+      for (int it = 0; it < T.nu; ++it) {
+        black();
+        step(solo);
+        red(false);
+        step(solo);
+      }
     }
+    __syncthreads();
   }
+}
+
+template <class KT, int kPairs>
+__global__ __launch_bounds__(kTailLanes) void k_tail_vcycle(TailCycle<KT> T) {
+  __shared__ TailStore S;
+  tail_load(T, S);
+  tail_cycle<KT, kPairs>(T, S);
+  for (int i = threadIdx.x; i < T.first[1] * 64; i += blockDim.x) T.lv[0].x[i] = S.x[i];
 }
 
 // y = A x in the edge-difference form.
@@ -1275,6 +1447,229 @@ __global__ void k_update_xr(uint64_t n, const float* d, const float* q, const fl
     v[3] += (rv / V) * (rv / V);
   }
   block_reduce(v, partial, blockIdx.x);
+}
+
+// ---- The whole iteration of a system whose level 0 is one of the small levels ----
+// One workgroup runs V-cycle, direction, step and the residual's norms, and tests convergence itself, in one
+// launch until the next restart. The iteration one launch at a time is seven launches, two copies and a wait
+// on the host around work of a few microseconds: a step of 24 blocks and six iterations takes 0.64 ms
+// instead of 1.00, a projection of as many 0.80 instead of 1.08. The sums are taken in the order of k_dot,
+// k_update_xr and the reductions that follow them (block partials, groups of four blocks, a tree over the
+// groups), so an iterate is the same bits on either path.
+struct SmallPcg {
+  const float *k, *diag, *vol;  // FP32 operator of level 0 (its anchors are the V-cycle's)
+  float *x, *r, *d, *q;
+  double* scal;
+  float* fscal;
+  uint64_t* err;
+  int budget;  // iterations of this launch at most
+  double integrated, volume, relative_defect;  // the last: the bound on the defect's norm, or negative
+};
+
+// Sum or maximum over the cells of a block, of values already combined over a lane's pair, ...
+template <bool kMax>
+__device__ inline double small_block(double v) {
+  for (int o = 16; o > 0; o >>= 1) v = kMax ? fmax(v, __shfl_xor(v, o)) : v + __shfl_xor(v, o);
+  return v;
+}
+// ... and over the blocks: every wave takes the whole reduction, one lane per group of four blocks.
+template <bool kMax>
+__device__ inline double small_total(const double* block) {
+  auto join = [](double a, double b) { return kMax ? fmax(a, b) : a + b; };
+  const double* g = block + 4 * (threadIdx.x & 15);
+  double v = join(join(join(g[0], g[1]), g[2]), g[3]);
+#pragma unroll
+  for (int s = 8; s > 0; s >>= 1) v = join(v, __shfl_down(v, s));
+  return __shfl(v, 0);
+}
+
+template <class KT, int kPairs>
+__global__ __launch_bounds__(kTailLanes) void k_small_pcg(TailCycle<KT> T, SmallPcg A) {
+  __shared__ TailStore S;
+  __shared__ double part[5][kTailBlocks];
+  __shared__ int bad;
+  constexpr int kZero = int(kTailBlocks) * 64;
+  const int t = threadIdx.x;
+  const int64_t n = int64_t(T.first[1]) * 64;
+  for (int i = t; i < 5 * int(kTailBlocks); i += blockDim.x) part[i / kTailBlocks][i % kTailBlocks] = 0.0;
+  if (t == 0) {
+    S.r[kZero] = 0.f;
+    bad = 0;
+  }
+  tail_load(T, S);
+  bool live[kPairs];
+  int at[kPairs];  // the red cell of each pair; the black one is 32 slots on
+  float x[kPairs][2], prev[kPairs][2], q[kPairs][2];
+#pragma unroll
+  for (int h = 0; h < kPairs; ++h) {
+    live[h] = tail_block(h) < T.first[1];
+    at[h] = tail_block(h) * 64 + (t & 31);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      x[h][c] = live[h] ? A.x[at[h] + 32 * c] : 0.f;
+      prev[h][c] = 0.f;
+      q[h][c] = 0.f;
+    }
+  }
+  double rho_prev = 0.0, rho = 0.0, curv = 0.0, l2 = 0.0, largest = 0.0, defect = 0.0;
+  float alpha = 0.f, beta = 0.f;
+  int done = 0, ordinal = -1, code = kOk;
+  while (done < A.budget) {
+    tail_cycle<KT, kPairs>(T, S);
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) {
+      double v = 0.0;
+      if (live[h])
+        v = static_cast<double>(S.b[at[h]]) * static_cast<double>(S.x[at[h]]) +
+            static_cast<double>(S.b[at[h] + 32]) * static_cast<double>(S.x[at[h] + 32]);
+      v = small_block<false>(v);
+      if (live[h] && (t & 31) == 0) part[0][tail_block(h)] = v;
+    }
+    __syncthreads();
+    rho = small_total<false>(part[0]);
+    if (!(rho > 0.0)) {
+      ordinal = 0;
+      code = kAborted;
+      break;
+    }
+    if (done > 0 && !fine_value(rho / rho_prev, beta)) {
+      ordinal = 1;
+      code = kOutOfRange;
+      break;
+    }
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h)
+      if (live[h])
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const float z = S.x[at[h] + 32 * c];
+          if (done > 0) {
+            const float keep = beta * prev[h][c];
+            prev[h][c] = z + keep;
+          } else {
+            prev[h][c] = z;
+          }
+          S.r[at[h] + 32 * c] = prev[h][c];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) {
+      double v = 0.0;
+      if (live[h]) {
+        const int blk = tail_block(h);
+        double w[2] = {0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          int sl = (c << 5) | (t & 31);
+          asm volatile("" : "+v"(sl));  // the 24 neighbour positions are formed here, not kept (and spilled) over the loop
+          const int l = cnat(sl), i = blk * 64 + sl;
+          const int pos[3] = {l & 3, (l >> 2) & 3, l >> 4};
+          const float di = prev[h][c];
+          float sum = T.lv[0].anchor[i] * di;
+#pragma unroll
+          for (int e = 0; e < 6; ++e) {
+            const int axis = e >> 1, step = 1 << (2 * axis);
+            const bool outside = pos[axis] == ((e & 1) ? 3 : 0);
+            const int nb = outside ? S.nbr[blk][e] : blk;
+            const int nl = (e & 1) ? (outside ? l - 3 * step : l + step) : (outside ? l + 3 * step : l - step);
+            const int j = nb >= 0 ? nb * 64 + cslot(nl) : kZero;
+            const int face = nb < 0 || !(e & 1) ? i : j;
+            float k;
+            if constexpr (std::is_same_v<KT, float>)
+              k = S.k[axis][face];
+            else
+              k = A.k[axis * n + face];
+            const float term = k * (di - S.r[j]);
+            if (nb >= 0) sum += term;
+          }
+          const bool unknown = A.diag[i] != 0.f;
+          q[h][c] = unknown ? sum : 0.f;
+          if (unknown) w[c] = static_cast<double>(di) * static_cast<double>(sum);
+        }
+        v = w[0] + w[1];
+      }
+      v = small_block<false>(v);
+      if (live[h] && (t & 31) == 0) part[1][tail_block(h)] = v;
+    }
+    __syncthreads();
+    curv = small_total<false>(part[1]);
+    if (!(curv > 0.0)) {
+      ordinal = 2;
+      code = kAborted;
+      break;
+    }
+    if (!fine_value(rho / curv, alpha)) {
+      ordinal = 3;
+      code = kOutOfRange;
+      break;
+    }
+    rho_prev = rho;
+#pragma unroll
+    for (int h = 0; h < kPairs; ++h) {
+      double u[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+      if (live[h])
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int i = at[h] + 32 * c;
+          if (A.diag[i] == 0.f) continue;
+          const float pi = alpha * prev[h][c];
+          const float fi = alpha * q[h][c];
+          const float xn = x[h][c] + pi;
+          const float rn = S.b[i] - fi;
+          if (!isfinite(xn) || !isfinite(rn)) {
+            perr_report(A.err + 1, 4, kOutOfRange);
+            bad = 1;
+          }
+          x[h][c] = xn;
+          S.b[i] = rn;
+          const double rv = rn, V = A.vol[i];
+          u[c][0] = rv * rv;
+          u[c][1] = fabs(rv) / V;
+          u[c][2] = (rv / V) * (rv / V);
+        }
+      const double s0 = small_block<false>(u[0][0] + u[1][0]);
+      const double s1 = small_block<true>(fmax(u[0][1], u[1][1]));
+      const double s2 = small_block<false>(u[0][2] + u[1][2]);
+      if (live[h] && (t & 31) == 0) {
+        part[2][tail_block(h)] = s0;
+        part[3][tail_block(h)] = s1;
+        part[4][tail_block(h)] = s2;
+      }
+    }
+    __syncthreads();
+    l2 = small_total<false>(part[2]);
+    largest = small_total<true>(part[3]);
+    defect = small_total<false>(part[4]);
+    ++done;
+    if (bad) break;
+    if (sqrt(l2) <= A.integrated && largest <= A.volume &&
+        (A.relative_defect < 0.0 || sqrt(defect) <= A.relative_defect))
+      break;
+  }
+#pragma unroll
+  for (int h = 0; h < kPairs; ++h)
+    if (live[h])
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int i = at[h] + 32 * c;
+        A.x[i] = x[h][c];
+        A.r[i] = S.b[i];
+        A.d[i] = prev[h][c];
+        A.q[i] = q[h][c];
+      }
+  if (t == 0) {
+    if (code != kOk) perr_report(A.err + 1, static_cast<uint64_t>(ordinal), code);
+    A.scal[0] = rho;
+    A.scal[1] = rho_prev;
+    A.scal[2] = curv;
+    A.scal[8] = l2;
+    A.scal[9] = largest;
+    A.scal[10] = 0.0;
+    A.scal[11] = defect;
+    A.scal[12] = done;
+    A.fscal[0] = alpha;
+    A.fscal[1] = beta;
+  }
 }
 
 // p = base + correction on the unknown cells.
@@ -1542,14 +1937,73 @@ LevelViewT<Bf16> view<Bf16>(Pressure& P, size_t l) {
           L.anchor,            L.diagb};
 }
 
+// The first level of the single-workgroup cycle: at most kTailBlocks blocks there, kTailStore in all, and
+// kMaxTail levels. The number of levels if there is none (a large coarsest level).
+size_t tail_start(const Pressure& P) {
+  size_t l = P.levels.size();
+  uint64_t blocks = 0;
+  while (l > 0 && P.levels[l - 1].nb <= kTailBlocks && blocks + P.levels[l - 1].nb <= uint64_t(kTailStore) &&
+         P.levels.size() - l < size_t(kMaxTail))
+    blocks += P.levels[--l].nb;
+  return l;
+}
+
+template <class KT>
+TailCycle<KT> tail_of(Pressure& P, size_t l, int nu, int coarse_sweeps) {
+  TailCycle<KT> T{};
+  T.count = static_cast<int>(P.levels.size() - l);
+  T.nu = nu;
+  T.coarse_sweeps = coarse_sweeps;
+  for (int q = 0; q < T.count; ++q) {
+    T.lv[q] = view<KT>(P, l + q);
+    T.first[q + 1] = T.first[q] + static_cast<int>(P.levels[l + q].nb);
+  }
+  return T;
+}
+
+// The widest small level, in blocks: 32 lanes per block, four waves at least (they load the levels), and two
+// pairs per lane where that is more than a workgroup.
+uint64_t tail_width(const Pressure& P, size_t l) {
+  uint64_t nb = 8;
+  for (; l < P.levels.size(); ++l) nb = std::max(nb, P.levels[l].nb);
+  return nb;
+}
+unsigned tail_lanes(uint64_t width) {
+  return static_cast<unsigned>(std::min<uint64_t>(kTailLanes, (32 * width + 63) / 64 * 64));
+}
+
+template <class KT>
+int run_tail(fl_ctx* ctx, Pressure& P, size_t l, int nu, int coarse_sweeps) {
+  const uint64_t width = tail_width(P, l);
+  const TailCycle<KT> T = tail_of<KT>(P, l, nu, coarse_sweeps);
+  if (32 * width > uint64_t(kTailLanes))
+    k_tail_vcycle<KT, 2><<<1, tail_lanes(width), 0, ctx->stream>>>(T);
+  else
+    k_tail_vcycle<KT, 1><<<1, tail_lanes(width), 0, ctx->stream>>>(T);
+  FL_HIP(hipGetLastError());
+  return FL_OK;
+}
+
+template <class KT>
+int run_small_pcg(fl_ctx* ctx, Pressure& P, int nu, int coarse_sweeps, const SmallPcg& A) {
+  const uint64_t width = tail_width(P, 0);
+  const TailCycle<KT> T = tail_of<KT>(P, 0, nu, coarse_sweeps);
+  if (32 * width > uint64_t(kTailLanes))
+    k_small_pcg<KT, 2><<<1, tail_lanes(width), 0, ctx->stream>>>(T, A);
+  else
+    k_small_pcg<KT, 1><<<1, tail_lanes(width), 0, ctx->stream>>>(T, A);
+  FL_HIP(hipGetLastError());
+  return FL_OK;
+}
+
 // V-cycle from level l. Level 0 smooths the recursive FP32 residual of the outer PCG in place of its
-// own right-hand side. Levels of at most kTailBlocks blocks (and everything below them) run in one
-// single-workgroup launch.
+// own right-hand side. The levels from tail_start on run in one single-workgroup launch.
 template <class KT>
 int vcycle(fl_ctx* ctx, Pressure& P, size_t l, int nu, int coarse_sweeps, int smoother) {
   hipStream_t s = ctx->stream;
   const size_t last = P.levels.size() - 1;
-  if (l == last && P.levels[l].nb > kTailBlocks) {  // a large coarsest level: grid-wide sweeps from zero
+  const size_t tail = tail_start(P);
+  if (l == last && l < tail) {  // a large coarsest level: grid-wide sweeps from zero
     const LevelViewT<KT> B = view<KT>(P, l);
     for (int pass = 0; pass < 4 * coarse_sweeps; ++pass) {
       const int fwd = pass < 2 * coarse_sweeps;
@@ -1558,17 +2012,7 @@ int vcycle(fl_ctx* ctx, Pressure& P, size_t l, int nu, int coarse_sweeps, int sm
     FL_HIP(hipGetLastError());
     return FL_OK;
   }
-  if (P.levels[l].nb <= kTailBlocks) {
-    TailCycle<KT> T{};
-    T.count = static_cast<int>(last - l + 1);
-    if (T.count > kMaxTail) return FL_INTERNAL;
-    T.nu = nu;
-    T.coarse_sweeps = coarse_sweeps;
-    for (size_t q = l; q <= last; ++q) T.lv[q - l] = view<KT>(P, q);
-    k_tail_vcycle<<<1, 1024, 0, s>>>(T);
-    FL_HIP(hipGetLastError());
-    return FL_OK;
-  }
+  if (l >= tail) return run_tail<KT>(ctx, P, l, nu, coarse_sweeps);
   if (smoother == 1 || (smoother == 2 && l > 0)) {  // block smoother: pre-smooth, restrict, coarse cycle, post
     const LevelViewT<KT> L = view<KT>(P, l), C = view<KT>(P, l + 1);
     const unsigned gb = static_cast<unsigned>((P.levels[l].nb + 3) / 4);
@@ -1647,6 +2091,8 @@ __global__ void k_reset_err(uint64_t* e) {
   if (threadIdx.x < 4) e[threadIdx.x] = ~uint64_t(0);
 }
 
+constexpr int kRestart = 10;  // iterations between restarts from the FP64 residual
+
 // The mixed-precision PCG with FP64 restarts. Requires the system to be frozen (faces, cells, RHS,
 // initial pressure in P.p_base) and the hierarchy coefficients set.
 int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates& gates, const EvalResult& zero_eval,
@@ -1699,7 +2145,10 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
   int stagnant = 0;
   double rn_prev = std::numeric_limits<double>::infinity();
   diag.learned_iterations = 0;
-  for (uint64_t it = 1; it <= opt.max_iterations; ++it) {
+  // A small system without the network (nor training pairs to collect) runs up to the next restart in one
+  // launch; the others one iteration at a time.
+  const bool small = tail_start(P) == 0 && !use_net && !(net && net->collect_every > 0);
+  auto iterate = [&](uint64_t it) -> int {
     if (use_net) {
       k_tile_gather<<<static_cast<unsigned>(P.ntiles), 512, 0, s>>>(P.r32, L0.diag, P.cell_class, P.tile_blocks,
                                                                     net->act, net->scale);
@@ -1737,6 +2186,18 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
                                         P.perr);
     k_finalize4<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, 8);
     FL_HIP(hipGetLastError());
+    return FL_OK;
+  };
+  for (uint64_t it = 1; it <= opt.max_iterations; ++it) {
+    if (small) {
+      const SmallPcg A{L0.k, L0.diag, P.fine_vol, P.x32, P.r32, P.d32, P.q32, P.scal, P.fscal, P.perr,
+                       static_cast<int>(std::min<uint64_t>(kRestart, opt.max_iterations - it + 1)), gates.integrated,
+                       gates.volume, gates.relative > 0.0 ? gates.relative * gates.initial_defect : -1.0};
+      FL_TRY(opt.level_storage == 2 ? run_small_pcg<Bf16>(ctx, P, opt.smoothing_sweeps, opt.coarse_sweeps, A)
+                                    : run_small_pcg<float>(ctx, P, opt.smoothing_sweeps, opt.coarse_sweeps, A));
+    } else {
+      FL_TRY(iterate(it));
+    }
     FL_HIP(hipMemcpyAsync(P.hscal, P.scal, 16 * sizeof(double), hipMemcpyDeviceToHost, s));
     FL_HIP(hipMemcpyAsync(ctx->host_words, P.perr, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     FL_HIP(hipStreamSynchronize(s));
@@ -1745,7 +2206,9 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
       return static_cast<int>(w & 0xff);
     }
     restart = false;
-    ++since;
+    const int done = small ? static_cast<int>(P.hscal[12]) : 1;
+    since += done;
+    it += static_cast<uint64_t>(done - 1);
     const double rn = std::sqrt(P.hscal[8]), rmax = P.hscal[9], dn = std::sqrt(P.hscal[11]);
     if (use_net) {
       stagnant = (rn > 0.9 * rn_prev || !(P.hscal[0] > 0.0)) ? stagnant + 1 : 0;
@@ -1758,7 +2221,7 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
     bool recursive = rn <= gates.integrated && rmax <= gates.volume;
     if (gates.relative > 0.0) recursive = recursive && dn <= gates.relative * gates.initial_defect;
     const bool last = it == opt.max_iterations;
-    if (!last && !recursive && since >= 10) {
+    if (!last && !recursive && since >= kRestart) {
       // Periodic restart from the FP64 true residual; acceptance is only tested at recursive
       // convergence or on the last iteration.
       k_apply_correction<<<grid_for(P.nc), kThreads, 0, s>>>(P.nc, P.cell_fine, P.cell_flag, P.p_base, P.x32, P.p,
@@ -1860,7 +2323,7 @@ int time_levels(fl_ctx* ctx, Pressure& P, int reps, fl_kernel_time* out, size_t 
     put(FL_KERNEL_RESTRICT_RED, 0, n0, ms);
     FL_TRY(mean_ms(ctx, reps, [&] { k_prolong<KT><<<grid_for(n0), kThreads, 0, s>>>(V0, P.levels[1].x); }, &ms));
     put(FL_KERNEL_PROLONG, 0, n0, ms);
-    if (P.levels[1].nb > kTailBlocks && P.levels.size() > 2) {
+    if (tail_start(P) > 1 && P.levels.size() > 2) {
       const LevelViewT<KT> V2 = view<KT>(P, 2);
       const unsigned gb = static_cast<unsigned>((P.levels[1].nb + 3) / 4);
       FL_TRY(mean_ms(ctx, reps, [&] { k_block_smooth<KT, false><<<gb, 256, 0, s>>>(V1, nullptr, nullptr, nu); }, &ms));
@@ -1877,20 +2340,10 @@ int time_levels(fl_ctx* ctx, Pressure& P, int reps, fl_kernel_time* out, size_t 
       put(FL_KERNEL_RESTRICT_ALL, 1, V1.n, ms);
     }
   }
-  // The single-workgroup tail from the first level of at most kTailBlocks blocks.
-  size_t first = P.levels.size();
-  for (size_t l = 0; l < P.levels.size(); ++l)
-    if (P.levels[l].nb <= kTailBlocks) {
-      first = l;
-      break;
-    }
-  if (first < P.levels.size() && P.levels.size() - first <= static_cast<size_t>(kMaxTail)) {
-    TailCycle<KT> T{};
-    T.count = static_cast<int>(P.levels.size() - first);
-    T.nu = nu;
-    T.coarse_sweeps = P.last_coarse_sweeps;
-    for (size_t q = first; q < P.levels.size(); ++q) T.lv[q - first] = view<KT>(P, q);
-    FL_TRY(mean_ms(ctx, reps, [&] { k_tail_vcycle<<<1, 1024, 0, s>>>(T); }, &ms));
+  // The single-workgroup cycle of the small levels.
+  const size_t first = tail_start(P);
+  if (first < P.levels.size()) {
+    FL_TRY(mean_ms(ctx, reps, [&] { (void)run_tail<KT>(ctx, P, first, nu, P.last_coarse_sweeps); }, &ms));
     put(FL_KERNEL_TAIL_VCYCLE, static_cast<uint32_t>(first), P.levels[first].nb * 64, ms);
   }
   // PCG kernels on level 0 (FP32 vectors and coefficients).

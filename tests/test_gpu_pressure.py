@@ -123,6 +123,29 @@ def test_bf16_level_storage_meets_the_same_gates(ctx):
     assert int(d["iteration_count"]) <= int(f32["diagnostics"]["iteration_count"]) + 3
 
 
+@pytest.mark.parametrize("anchored,bf16", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("minimum,extents,levels", [(0, (1, 1, 2), 2), (0, (4, 4, 3), 3), (0, (8, 4, 4), 3),
+                                                    (0, (12, 4, 4), 4), (-3, (7, 5, 6), 16), (0, (16, 15, 8), 3),
+                                                    (0, (16, 12, 11), 3), (0, (16, 16, 16), 2), (0, (16, 16, 16), 3),
+                                                    (0, (19, 16, 16), 3), (-1, (10, 9, 5), 1)])
+def test_small_systems_meet_the_affine_solution(ctx, minimum, extents, levels, anchored, bf16):
+    # One block, one wave's two blocks, three blocks, sixteen levels, 32 blocks (the last with one cell pair per
+    # lane), 36, 64 with 8 below (all of whose iterations run in one launch), 64 with 8 and 1 (also), 80 (a
+    # larger level above the small ones), and one level only; the target needs restarts. The relative target bounds the defect by 1e-10 of its initial norm (below 1e2 here);
+    # the inverse operator is below (21 / pi)^2 and a pressure differs by at most that times the defect: 5e-7.
+    geom, sb, cells, faces, pressure = K.affine_problem(minimum, extents, anchored)
+    s, out = ctx.project(geom, sb, 1.0, cells, faces,
+                         H.pressure_options(relative_target=1e-10, levels=levels, coarse_sweeps=4, bf16_levels=bf16))
+    assert s == H.OK, s
+    d = out["diagnostics"]
+    print("iterations", d["iteration_count"], "restarts", d["restarts"], "levels", d["multigrid_level_count"], flush=True)
+    want = np.array([pressure(tuple(c)) for c in cells["cell_index"].tolist()])
+    if not anchored:
+        want -= want[out["gauges"][0]]
+    np.testing.assert_allclose(out["pressures"], want, atol=5e-7)
+    np.testing.assert_allclose(out["velocities"], 0.0, atol=5e-7)
+
+
 @pytest.mark.parametrize("bf16,smoother", [(False, 1), (True, 1), (True, 2)], ids=["fp32_block", "bf16_block",
                                                                                "bf16_hybrid"])
 def test_block_smoother_meets_the_gates_deterministically(ctx, bf16, smoother):
