@@ -69,6 +69,7 @@ struct Level {
   float* k = nullptr;       // [3][nb*64] low-face conductances along x, y, z
   float* anchor = nullptr;  // [nb*64]
   float* diag = nullptr;    // [nb*64], 0 marks a non-unknown cell
+  const int32_t* tiles = nullptr;  // [coarser blocks][128] for the tile smoother, or null
 };
 
 struct Pressure {
@@ -135,6 +136,8 @@ struct Pressure {
   // Multigrid level storage: one device pool reserved with the other arrays, carved level by level.
   unsigned char* level_pool = nullptr;
   uint64_t pool_bytes = 0, pool_used = 0;
+  int32_t* tile_table = nullptr;  // [cap_tiles][128]: Level::tiles
+  uint64_t cap_tiles = 0;
   int levels_requested = 0;
   int last_storage = 1, last_nu = 2, last_coarse_sweeps = 2;  // V-cycle settings of the last solve
   bool p_init_zero = false;  // warm start is identically zero: its evaluation equals the p = 0 one
@@ -930,6 +933,220 @@ __global__ void k_restrict_all(const float* r, LevelViewT<KT> C) {
     sum += r[uint64_t(fb) * 64 + cslot((fz & 3) * 16 + (fy & 3) * 4 + (fx & 3))];
   }
   const_cast<float*>(C.b)[i] = sum;
+}
+
+// ---- Level-wide smoothing by tiles: up to four half sweeps in one launch ----
+// A half sweep over a level of a few thousand blocks is a launch of 4 us in which the chip does little, and
+// the half sweeps of a smoothing step wait for each other. A tile is the 8^3 cells under one coarse block;
+// its workgroup copies the tile and a halo of four cells (two for one sweep) into LDS and takes the half
+// sweeps there, each over a cube smaller by one cell on every side than the one before, so that the last
+// one covers the tile: the values in the halo are recomputed, from the same terms in the same order, by
+// every tile that needs them, and the result is the level-wide sweeps' bit for bit. The coefficients of all
+// the half sweeps are requested at once, before the first one. Two sweeps recompute 2.9 times as many cells
+// as they produce: with 160 tiles (a workgroup for most of the CUs) they take 10 us with the correction and
+// 6.7 from zero where four launches and the correction's took 20 and 16; a step of 1120 blocks (160 and 24
+// tiles) takes 1.88 ms instead of 2.52, one of 5712 (714 tiles; three sweeps) 6.27 instead of 6.78, one of 8320
+// (1120 tiles) 5.84 instead of 5.60, so the half sweeps stay apart from about three tiles per CU on.
+constexpr int kTileLanes = 512;
+constexpr uint64_t kTileLimit = 768;             // tiles of a level
+constexpr uint64_t kTileTable = 2 * kTileLimit;  // tiles of all levels of a hierarchy
+
+// Tile tables, one wave per coarse block: the level's blocks in the 4^3 around the tile's eight ((z,y,x)
+// order, -1 where there is none or none that a path of face neighbours from the tile leads to), then their
+// coarser blocks. Blocks without a coarse parent (no unknowns) belong to no tile: their values are zeroed here,
+// in both buffers.
+__global__ __launch_bounds__(256) void k_tile_table(const int32_t* nbr, const int32_t* parent, uint64_t nb,
+                                                    const int32_t* child, uint64_t tiles, int32_t* table, float* x,
+                                                    float* r) {
+  __shared__ int ids[4][64];
+  const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+  const uint64_t c = blockIdx.x * 4ull + w;
+  if (c < nb && parent[2 * c] < 0) {
+    x[64 * c + t] = 0.f;
+    r[64 * c + t] = 0.f;
+  }
+  const int bx = t & 3, by = (t >> 2) & 3, bz = t >> 4;
+  const bool inner = (bx == 1 || bx == 2) && (by == 1 || by == 2) && (bz == 1 || bz == 2);
+  int id = -1;
+  if (inner && c < tiles) id = child[8 * c + ((bz - 1) * 2 + (by - 1)) * 2 + (bx - 1)];
+  for (int round = 0; round < 3; ++round) {
+    ids[w][t] = id;
+    __syncthreads();
+    if (id < 0) {
+      const int at[3] = {bx, by, bz};
+      for (int dir = 0; dir < 6 && id < 0; ++dir) {
+        const int axis = dir >> 1, to = at[axis] + ((dir & 1) ? 1 : -1);
+        if (to < 0 || to > 3) continue;
+        const int from = ids[w][t + ((dir & 1) ? 1 : -1) * (1 << (2 * axis))];
+        if (from >= 0) id = nbr[6 * from + (dir ^ 1)];
+      }
+    }
+    __syncthreads();
+  }
+  if (c >= tiles) return;
+  table[128 * c + t] = id;
+  table[128 * c + 64 + t] = id < 0 ? -1 : parent[2 * id];
+}
+
+// The cells of one colour of a cube of side S about the tile, in local coordinates [0, 16)^3 with the tile at
+// [4, 12)^3. In LDS the colours are apart, each row of 16 cells as eight: position (z * 16 + y) * 8 + x / 2.
+template <class KT, int S>
+struct TileStage {
+  static constexpr int kCells = S * S * S / 2, kRounds = (kCells + kTileLanes - 1) / kTileLanes, kLow = 8 - S / 2;
+  float d[kRounds], b[kRounds], k[kRounds][6];
+  int at[kRounds];  // LDS position * 2 + (x odd), or -1
+
+  // Calls f(round, x, y, z) for the lane's cells of `colour`.
+  template <class F>
+  static __device__ inline void cells(int colour, F f) {
+#pragma unroll
+    for (int q = 0; q < kRounds; ++q) {
+      const int e = q * kTileLanes + threadIdx.x;
+      if (e >= kCells) continue;
+      const int row = e / (S / 2), y = kLow + row % S, z = kLow + row / S;
+      const int x = kLow + 2 * (e % (S / 2)) + ((colour + kLow + y + z) & 1);
+      f(q, x, y, z);
+    }
+  }
+  __device__ inline void load(const LevelViewT<KT>& L, const int* ids, int colour, bool coefficients) {
+#pragma unroll
+    for (int q = 0; q < kRounds; ++q) at[q] = -1;
+    cells(colour, [&](int q, int x, int y, int z) {
+      at[q] = (((z * 16 + y) * 8 + (x >> 1)) << 1) | (x & 1);
+      d[q] = 0.f;
+      b[q] = 0.f;
+#pragma unroll
+      for (int dir = 0; dir < 6; ++dir) k[q][dir] = 0.f;
+      const int slot = (z >> 2) * 16 + (y >> 2) * 4 + (x >> 2), id = ids[slot];
+      if (id < 0) return;
+      // The colour half of a slot is known: the cell's own is `colour`, its neighbours' the other one.
+      const int l = (z & 3) * 16 + (y & 3) * 4 + (x & 3);
+      const uint32_t n = static_cast<uint32_t>(L.n), g = uint32_t(id) * 64 + ((colour << 5) | (l >> 1));
+      d[q] = L.diag[g];
+      b[q] = L.b[g];
+      if (!coefficients) return;
+      const int pos[3] = {x & 3, y & 3, z & 3};
+#pragma unroll
+      for (int axis = 0; axis < 3; ++axis) {
+        const int step = 1 << (2 * axis);
+        const bool outside = pos[axis] == 3;
+        const int nid = outside ? ids[slot + step] : id;
+        const uint32_t j = uint32_t(nid) * 64 + (((1 - colour) << 5) | ((outside ? l - 3 * step : l + step) >> 1));
+        k[q][2 * axis] = kload(L.k, axis * n + g);  // zero where no block lies below
+        if (nid >= 0) k[q][2 * axis + 1] = kload(L.k, axis * n + j);
+      }
+    });
+  }
+  __device__ inline void run(float (*xs)[2048], int colour, bool zero) const {
+#pragma unroll
+    for (int q = 0; q < kRounds; ++q) {
+      if (at[q] < 0) continue;
+      const int p = at[q] >> 1, odd = at[q] & 1;
+      float s = b[q];
+      if (!zero) {
+        const float* o = xs[1 - colour];
+        const float xx[6] = {o[p - 1 + odd], o[p + odd], o[p - 8], o[p + 8], o[p - 128], o[p + 128]};
+#pragma unroll
+        for (int dir = 0; dir < 6; ++dir) s += k[q][dir] * xx[dir];
+      }
+      xs[colour][p] = d[q] == 0.f ? 0.f : s / d[q];
+    }
+  }
+};
+
+// kSweeps sweeps (two half sweeps each). kZero: from zero, red first, into L.x itself; otherwise from L.x, with
+// the coarse correction xc added first if kCorrect, black first if kPost, into the second buffer.
+template <class KT, int kSweeps, bool kZero, bool kPost, bool kCorrect>
+__global__ __launch_bounds__(kTileLanes) void k_tile_smooth(LevelViewT<KT> L, const int32_t* tiles, float* out,
+                                                            const float* xc) {
+  __shared__ float xs[2][2048];
+  __shared__ int ids[128];
+  constexpr int c0 = kPost ? 1 : 0;
+  const int t = threadIdx.x;
+  if (t < 128) ids[t] = tiles[128 * uint64_t(blockIdx.x) + t];
+  __syncthreads();
+  TileStage<KT, 14> A;
+  TileStage<KT, 12> B;
+  TileStage<KT, 10> C;
+  TileStage<KT, 8> D;
+  if constexpr (!kZero)
+    TileStage<KT, kSweeps == 2 ? 16 : 12>::cells(1 - c0, [&](int, int x, int y, int z) {
+      const int slot = (z >> 2) * 16 + (y >> 2) * 4 + (x >> 2), id = ids[slot];
+      float v = 0.f;
+      if (id >= 0) {
+        const uint32_t g = uint32_t(id) * 64 + (((1 - c0) << 5) | (((z & 3) * 16 + (y & 3) * 4 + (x & 3)) >> 1));
+        v = L.x[g];
+        if constexpr (kCorrect)
+          if (L.diag[g] != 0.f)  // the tile starts at a coarse block: coarse cell (c - 4) / 2 of it or a neighbour
+            v += xc[uint64_t(ids[64 + slot]) * 64 +
+                    cslot((((z + 4) >> 1) & 3) * 16 + (((y + 4) >> 1) & 3) * 4 + (((x + 4) >> 1) & 3))];
+      }
+      xs[1 - c0][(z * 16 + y) * 8 + (x >> 1)] = v;
+    });
+  if constexpr (kSweeps == 2) {
+    A.load(L, ids, c0, !kZero);
+    B.load(L, ids, 1 - c0, true);
+  }
+  C.load(L, ids, c0, kSweeps == 2 || !kZero);
+  D.load(L, ids, 1 - c0, true);
+  __syncthreads();
+  if constexpr (kSweeps == 2) {
+    A.run(xs, c0, kZero);
+    __syncthreads();
+    B.run(xs, 1 - c0, false);
+    __syncthreads();
+  }
+  C.run(xs, c0, kZero && kSweeps == 1);
+  __syncthreads();
+  D.run(xs, 1 - c0, false);
+  __syncthreads();
+  const int octant = t >> 6, sl = t & 63, l = cnat(sl);
+  const int bx = 1 + (octant & 1), by = 1 + ((octant >> 1) & 1), bz = 1 + (octant >> 2);
+  const int id = ids[bz * 16 + by * 4 + bx];
+  if (id < 0) return;
+  const int x = 4 * bx + (l & 3), y = 4 * by + ((l >> 2) & 3), z = 4 * bz + (l >> 4);
+  out[uint64_t(id) * 64 + sl] = xs[sl >> 5][(z * 16 + y) * 8 + (x >> 1)];
+}
+
+// Residual of the red cells after pre-smoothing and its sum over the children in one pass: one workgroup per
+// coarse block, one lane per red fine cell, the four of a coarse cell side by side.
+template <class KT>
+__global__ __launch_bounds__(256) void k_residual_restrict(LevelViewT<KT> F, LevelViewT<KT> C) {
+  const int t = threadIdx.x, octant = t >> 5, cell = (t >> 2) & 7;
+  const int o = (t & 3) == 0 ? 0 : (t & 3) == 1 ? 3 : (t & 3) == 2 ? 5 : 6;  // even octants: the red children
+  const uint64_t c = blockIdx.x;
+  const int32_t fb = C.child[8 * c + octant];
+  float r = 0.f;
+  if (fb >= 0) {
+    const int lx = 2 * (cell & 1) + (o & 1), ly = 2 * ((cell >> 1) & 1) + ((o >> 1) & 1),
+              lz = 2 * (cell >> 2) + (o >> 2);
+    const uint64_t i = uint64_t(fb) * 64 + cslot(lz * 16 + ly * 4 + lx);
+    const float xi = F.x[i], anchor = F.anchor[i], b = F.b[i], d = F.diag[i];
+    float kk[6], xx[6];
+    bool there[6];
+#pragma unroll
+    for (int dir = 0; dir < 6; ++dir) {
+      const int64_t j = neighbour(F.nbr, uint64_t(fb), lx, ly, lz, dir);
+      there[dir] = j >= 0;
+      const int64_t jj = j < 0 ? static_cast<int64_t>(i) : j;
+      kk[dir] = face_kt(F.k, F.n, static_cast<int64_t>(i), jj, dir);
+      xx[dir] = F.x[jj];
+    }
+    float a = anchor * xi;
+#pragma unroll
+    for (int dir = 0; dir < 6; ++dir) {
+      const float term = kk[dir] * (xi - xx[dir]);
+      if (there[dir]) a += term;
+    }
+    r = d == 0.f ? 0.f : b - a;
+  }
+  const int lane = t & 63 & ~3;
+  float sum = 0.f;
+  for (int q = 0; q < 4; ++q) sum += __shfl(r, lane + q);
+  if ((t & 3) != 0) return;
+  const int x = 2 * (octant & 1) + (cell & 1), y = 2 * ((octant >> 1) & 1) + ((cell >> 1) & 1),
+            z = 2 * (octant >> 2) + (cell >> 2);
+  const_cast<float*>(C.b)[64 * c + cslot(z * 16 + y * 4 + x)] = sum;
 }
 
 // ---- The small levels, in one workgroup with every value in LDS ----
@@ -1728,6 +1945,7 @@ int ensure_capacity(fl_ctx* ctx, uint64_t nc, uint64_t nf, uint64_t nfine) {
   dfree(P.level_pool);
   P.pool_bytes = 0;
   dfree(P.tile_blocks);
+  dfree(P.tile_table);
   dfree(P.cell_class);
   P.ntiles = 0;
   void* ptrs[] = {P.fine_cell, P.cell_fine, P.cell_flag, P.cell_faces, P.face_tail, P.face_head, P.face_kind,
@@ -1766,6 +1984,8 @@ int ensure_capacity(fl_ctx* ctx, uint64_t nc, uint64_t nf, uint64_t nfine) {
   FL_TRY(dal(&P.fine_vol, cn));
   FL_TRY(dal(&P.cell_class, cn));
   FL_TRY(dal(&P.tile_blocks, 8 * (cn / 64)));
+  P.cap_tiles = std::min<uint64_t>(cn / 64, kTileTable);
+  FL_TRY(dal(&P.tile_table, 128 * P.cap_tiles));
   FL_TRY(dal(&P.r32, cn));
   FL_TRY(dal(&P.x32, cn));
   FL_TRY(dal(&P.d32, cn));
@@ -1898,6 +2118,17 @@ int build_levels(fl_ctx* ctx, Pressure& P, const std::vector<Key3>& blocks0, int
   return FL_OK;
 }
 
+// The first level of the single-workgroup cycle: at most kTailBlocks blocks there, kTailStore in all, and
+// kMaxTail levels. The number of levels if there is none (a large coarsest level).
+size_t tail_start(const Pressure& P) {
+  size_t l = P.levels.size();
+  uint64_t blocks = 0;
+  while (l > 0 && P.levels[l - 1].nb <= kTailBlocks && blocks + P.levels[l - 1].nb <= uint64_t(kTailStore) &&
+         P.levels.size() - l < size_t(kMaxTail))
+    blocks += P.levels[--l].nb;
+  return l;
+}
+
 // Level coefficients from the links' conductances (or from `conductance` when given: the coupled
 // viscous solve's effective conductances).
 int setup_coefficients(fl_ctx* ctx, Pressure& P, const double* conductance = nullptr) {
@@ -1920,6 +2151,19 @@ int setup_coefficients(fl_ctx* ctx, Pressure& P, const double* conductance = nul
     k_diag<<<grid_for(ncc), kThreads, 0, s>>>(ncc, C.nbr, C.k, C.anchor, C.diag);
     FL_HIP(hipGetLastError());
   }
+  uint64_t used = 0;
+  for (size_t l = 0; l + 1 < P.levels.size(); ++l) {
+    Level& F = P.levels[l];
+    const Level& C = P.levels[l + 1];
+    F.tiles = nullptr;
+    if (l >= tail_start(P) || C.nb > kTileLimit || used + C.nb > P.cap_tiles) continue;
+    int32_t* table = P.tile_table + 128 * used;
+    used += C.nb;
+    k_tile_table<<<static_cast<unsigned>((std::max(F.nb, C.nb) + 3) / 4), 256, 0, s>>>(F.nbr, F.parent, F.nb, C.child,
+                                                                                     C.nb, table, F.x, F.r);
+    FL_HIP(hipGetLastError());
+    F.tiles = table;
+  }
   return FL_OK;
 }
 
@@ -1935,17 +2179,6 @@ LevelViewT<Bf16> view<Bf16>(Pressure& P, size_t l) {
   Level& L = P.levels[l];
   return {L.nb * 64,           L.nbr,  L.child, L.parent, L.x, l == 0 ? P.r32 : L.b, reinterpret_cast<const Bf16*>(L.kb),
           L.anchor,            L.diagb};
-}
-
-// The first level of the single-workgroup cycle: at most kTailBlocks blocks there, kTailStore in all, and
-// kMaxTail levels. The number of levels if there is none (a large coarsest level).
-size_t tail_start(const Pressure& P) {
-  size_t l = P.levels.size();
-  uint64_t blocks = 0;
-  while (l > 0 && P.levels[l - 1].nb <= kTailBlocks && blocks + P.levels[l - 1].nb <= uint64_t(kTailStore) &&
-         P.levels.size() - l < size_t(kMaxTail))
-    blocks += P.levels[--l].nb;
-  return l;
 }
 
 template <class KT>
@@ -2025,6 +2258,41 @@ int vcycle(fl_ctx* ctx, Pressure& P, size_t l, int nu, int coarse_sweeps, int sm
     k_block_smooth<KT, true><<<gb, 256, 0, s>>>(Lp, P.levels[l].r, P.levels[l + 1].x, nu);
     FL_HIP(hipGetLastError());
     std::swap(P.levels[l].x, P.levels[l].r);  // the post-smoothed values are the level's x from here on
+    return FL_OK;
+  }
+  if (P.levels[l].tiles) {
+    const unsigned tiles = static_cast<unsigned>(P.levels[l + 1].nb);
+    const int32_t* table = P.levels[l].tiles;
+    Level& F = P.levels[l];
+    // Two sweeps to a launch, the odd one last; every launch but the one from zero swaps the buffers.
+    if (nu >= 2)
+      k_tile_smooth<KT, 2, true, false, false><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.x, nullptr);
+    else
+      k_tile_smooth<KT, 1, true, false, false><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.x, nullptr);
+    for (int done = 2; done < nu; done += 2) {
+      if (nu - done >= 2)
+        k_tile_smooth<KT, 2, false, false, false><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.r, nullptr);
+      else
+        k_tile_smooth<KT, 1, false, false, false><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.r, nullptr);
+      std::swap(F.x, F.r);
+    }
+    k_residual_restrict<<<tiles, 256, 0, s>>>(view<KT>(P, l), view<KT>(P, l + 1));
+    FL_HIP(hipGetLastError());
+    FL_TRY(vcycle<KT>(ctx, P, l + 1, nu, coarse_sweeps, smoother));
+    const float* xc = P.levels[l + 1].x;
+    if (nu >= 2)
+      k_tile_smooth<KT, 2, false, true, true><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.r, xc);
+    else
+      k_tile_smooth<KT, 1, false, true, true><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.r, xc);
+    std::swap(F.x, F.r);
+    for (int done = 2; done < nu; done += 2) {
+      if (nu - done >= 2)
+        k_tile_smooth<KT, 2, false, true, false><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.r, nullptr);
+      else
+        k_tile_smooth<KT, 1, false, true, false><<<tiles, kTileLanes, 0, s>>>(view<KT>(P, l), table, F.r, nullptr);
+      std::swap(F.x, F.r);
+    }
+    FL_HIP(hipGetLastError());
     return FL_OK;
   }
   const LevelViewT<KT> L = view<KT>(P, l), C = view<KT>(P, l + 1);
@@ -2263,6 +2531,7 @@ void destroy_pressure(fl_ctx* ctx) {
   free_levels(*P);
   dfree(P->level_pool);
   dfree(P->tile_blocks);
+  dfree(P->tile_table);
   dfree(P->cell_class);
   void* ptrs[] = {P->fine_cell, P->cell_fine, P->cell_flag, P->cell_faces, P->face_tail, P->face_head, P->face_kind,
                   P->face_slot, P->face_area, P->face_beta, P->face_dist, P->face_ustar, P->face_uwall, P->face_flux,

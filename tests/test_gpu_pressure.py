@@ -146,6 +146,24 @@ def test_small_systems_meet_the_affine_solution(ctx, minimum, extents, levels, a
     np.testing.assert_allclose(out["velocities"], 0.0, atol=5e-7)
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("sweeps", [1, 2, 3, 5])
+@pytest.mark.parametrize("minimum,extents", [(0, (19, 16, 16)), (-5, (27, 13, 25)), (3, (64, 9, 9))])
+def test_level_wide_sweeps_by_tiles(ctx, minimum, extents, sweeps, bf16):
+    # Levels above the small ones, smoothed by tiles: one and two sweeps to a launch, odd numbers, boxes that begin
+    # inside a block, an odd block of a tile, and a row of tiles. With FP32 and BF16 coefficients alike (they are 1
+    # and exact in BF16), and bounded like the small systems: at 64 cells (64 / pi)^2 1e-8 < 5e-6.
+    geom, sb, cells, faces, pressure = K.affine_problem(minimum, extents, True)
+    s, out = ctx.project(geom, sb, 1.0, cells, faces,
+                         H.pressure_options(relative_target=1e-10, levels=4, sweeps=sweeps, coarse_sweeps=4,
+                                            bf16_levels=bf16))
+    assert s == H.OK, s
+    print("iterations", out["diagnostics"]["iteration_count"], flush=True)
+    want = np.array([pressure(tuple(c)) for c in cells["cell_index"].tolist()])
+    np.testing.assert_allclose(out["pressures"], want, atol=5e-6)
+    np.testing.assert_allclose(out["velocities"], 0.0, atol=5e-6)
+
+
 @pytest.mark.parametrize("bf16,smoother", [(False, 1), (True, 1), (True, 2)], ids=["fp32_block", "bf16_block",
                                                                                "bf16_hybrid"])
 def test_block_smoother_meets_the_gates_deterministically(ctx, bf16, smoother):
