@@ -167,11 +167,19 @@ __global__ __launch_bounds__(256) void k_mark_candidates_bins(const double* sx, 
     if (!ok) continue;
     if (inside) {
       for (int32_t z = lo[2]; z <= hi[2]; ++z)
-        for (int32_t y = lo[1]; y <= hi[1]; ++y)
-          for (int32_t x = lo[0]; x <= hi[0]; ++x) {
-            const int b = ((z - w0[2]) * W + (y - w0[1])) * W + (x - w0[0]);
-            atomicOr(&win[b >> 5], 1u << (b & 31));
+        for (int32_t y = lo[1]; y <= hi[1]; ++y) {
+          // A row of cells at a time, and only where a bit is missing (most are there: a bin's particles cover
+          // nearly the same cells): an LDS atomic per cell and particle took 0.28 ms for 4.5 million particles,
+          // this 0.09.
+          for (int b = ((z - w0[2]) * W + (y - w0[1])) * W + (lo[0] - w0[0]), left = hi[0] - lo[0] + 1; left > 0;) {
+            const int word = b >> 5, in = min(left, 32 - (b & 31));
+            const unsigned int mask = (in == 32 ? ~0u : (1u << in) - 1u) << (b & 31);
+            if ((__hip_atomic_load(&win[word], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & mask) != mask)
+              atomicOr(&win[word], mask);
+            b += in;
+            left -= in;
           }
+        }
     } else {
       for (int32_t z = lo[2]; z <= hi[2]; ++z)
         for (int32_t y = lo[1]; y <= hi[1]; ++y) {
