@@ -31,6 +31,7 @@ namespace {
 
 constexpr double kEpsD = 2.220446049250313080847e-16;
 constexpr int kPartials = 16384;  // reduction partial slots (one per workgroup of a reducing kernel)
+constexpr int kHostErrors = 32;  // the error words in the pinned mirror of the scalars
 constexpr unsigned kStreamPartials = 2048;  // workgroups of the grid-stride streaming reductions
 
 struct Key3 {
@@ -558,7 +559,11 @@ __global__ void k_rhs_zero_eval(uint64_t nc, const int32_t* cell_faces, const Fa
 
 
 // Reduces the 4 partial rows in a fixed order into scal[base..base+3].
-__global__ void k_finalize4(const double* partial, unsigned slots, double* scal, int base) {
+// host: when set, what the host looks at (these four values, rho, the handover mark and the two error words) goes
+// straight to its pinned mirror. As two copies per iteration and evaluation, 3 us each with the gaps around
+// them, it was 5 % of a step of 1120 blocks and 12 iterations.
+__global__ void k_finalize4(const double* partial, unsigned slots, double* scal, int base, double* host,
+                            const uint64_t* err) {
   __shared__ double red[4][kThreads];
   double a = 0.0, b = 0.0, c = 0.0, d = 0.0;
   for (unsigned i = threadIdx.x; i < slots; i += blockDim.x) {
@@ -581,8 +586,15 @@ __global__ void k_finalize4(const double* partial, unsigned slots, double* scal,
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0)
+  if (threadIdx.x == 0) {
     for (int q = 0; q < 4; ++q) scal[base + q] = red[q][0];
+    if (host) {
+      for (int q = 0; q < 4; ++q) host[base + q] = red[q][0];
+      host[0] = scal[0];
+      host[14] = scal[14];
+      for (int q = 0; q < 2; ++q) reinterpret_cast<uint64_t*>(host)[kHostErrors + q] = err[q];
+    }
+  }
 }
 
 // ------------------------------------------------------------------ level coefficients
@@ -2326,17 +2338,17 @@ struct EvalResult {
 // Reduces the evaluation partials of `groups` workgroups and reads the norms and error words back.
 int read_evaluation(fl_ctx* ctx, Pressure& P, unsigned g, EvalResult& out) {
   hipStream_t s = ctx->stream;
-  k_finalize4<<<1, kThreads, 0, s>>>(P.partial, g, P.scal, 8);
+  k_finalize4<<<1, kThreads, 0, s>>>(P.partial, g, P.scal, 8, P.hscal, P.perr);
   FL_HIP(hipGetLastError());
-  FL_HIP(hipMemcpyAsync(P.hscal, P.scal, 16 * sizeof(double), hipMemcpyDeviceToHost, s));
-  FL_HIP(hipMemcpyAsync(ctx->host_words, P.perr, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   FL_HIP(hipStreamSynchronize(s));
+  uint64_t words[2];
+  std::memcpy(words, P.hscal + kHostErrors, sizeof(words));
   out.l2 = std::sqrt(P.hscal[8]);
   out.max_res = P.hscal[9];
   out.max_def = P.hscal[10];
   out.def_l2 = std::sqrt(P.hscal[11]);
-  out.code = ctx->host_words[0] != ~uint64_t(0) ? static_cast<int>(ctx->host_words[0] & 0xff) : FL_OK;
-  if (out.code == FL_OK && ctx->host_words[1] != ~uint64_t(0)) out.code = static_cast<int>(ctx->host_words[1] & 0xff);
+  out.code = words[0] != ~uint64_t(0) ? static_cast<int>(words[0] & 0xff) : FL_OK;
+  if (out.code == FL_OK && words[1] != ~uint64_t(0)) out.code = static_cast<int>(words[1] & 0xff);
   return FL_OK;
 }
 
@@ -2442,7 +2454,7 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
     }
     if (use_net && !restart) {  // z . q_prev for the flexible-CG orthogonalisation, before q is overwritten
       k_dot<<<rg, kThreads, 0, s>>>(n, L0.x, P.q32, P.partial);
-      k_finalize4<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, 28);
+      k_finalize4<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, 28, nullptr, nullptr);
     }
     k_dot<<<rg, kThreads, 0, s>>>(n, P.r32, L0.x, P.partial);
     k_finalize_step<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, P.fscal, P.perr, use_net ? 2 : 1, restart ? 1 : 0);
@@ -2452,7 +2464,7 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
     k_finalize_step<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, P.fscal, P.perr, use_net ? 4 : 3, 0);
     k_update_xr<<<rg, kThreads, 0, s>>>(n, P.d32, P.q32, L0.diag, P.fine_vol, P.x32, P.r32, P.fscal, P.partial,
                                         P.perr);
-    k_finalize4<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, 8);
+    k_finalize4<<<1, kThreads, 0, s>>>(P.partial, rg, P.scal, 8, P.hscal, P.perr);
     FL_HIP(hipGetLastError());
     return FL_OK;
   };
@@ -2463,16 +2475,15 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
                        gates.volume, gates.relative > 0.0 ? gates.relative * gates.initial_defect : -1.0};
       FL_TRY(opt.level_storage == 2 ? run_small_pcg<Bf16>(ctx, P, opt.smoothing_sweeps, opt.coarse_sweeps, A)
                                     : run_small_pcg<float>(ctx, P, opt.smoothing_sweeps, opt.coarse_sweeps, A));
+      FL_HIP(hipMemcpyAsync(P.hscal, P.scal, 16 * sizeof(double), hipMemcpyDeviceToHost, s));
+      FL_HIP(hipMemcpyAsync(P.hscal + kHostErrors, P.perr, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     } else {
       FL_TRY(iterate(it));
     }
-    FL_HIP(hipMemcpyAsync(P.hscal, P.scal, 16 * sizeof(double), hipMemcpyDeviceToHost, s));
-    FL_HIP(hipMemcpyAsync(ctx->host_words, P.perr, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     FL_HIP(hipStreamSynchronize(s));
-    if (ctx->host_words[1] != ~uint64_t(0)) {
-      const uint64_t w = ctx->host_words[1];
-      return static_cast<int>(w & 0xff);
-    }
+    uint64_t words[2];
+    std::memcpy(words, P.hscal + kHostErrors, sizeof(words));
+    if (words[1] != ~uint64_t(0)) return static_cast<int>(words[1] & 0xff);
     restart = false;
     const int done = small ? static_cast<int>(P.hscal[12]) : 1;
     since += done;
