@@ -19,6 +19,7 @@
 // other particle can hold the minimum, and the result equals the reference's scan over all
 // particles bit for bit (min is exact and order-free).
 #include "context.h"
+#include "ring_walk.h"
 #include "stdmath.h"
 
 namespace fl {
@@ -354,9 +355,7 @@ struct SubGrid {
 // the index), world position origin + lattice * h as the reference rounds it. One pass keeps the least
 // squared distance d2 and the least hypot among the particles whose d2 is within a relative 1e-10 of
 // it: a particle more than that above the least d2 is farther than the hypot minimum by far more than
-// hypot's rounding. Sub-cells are visited in rings of growing radius rho (cells); within a ring a
-// sub-cell whose box is farther than the current least distance is skipped, and the search ends when
-// every unvisited sub-cell lies beyond the least distance. Bound by the walk over sub-cells, not by the
+// hypot's rounding. ring_walk.h visits the sub-cells. Bound by the walk over sub-cells, not by the
 // particles' loads or the hypot (batches of loads, a hypot put off to the end and eight lanes per sample
 // were no faster or slower): the samples around the surface, whose nearest particle lies beyond two cells,
 // took rings of four cells, 2,000 sub-cells in two passes. Centres and corners share a launch, whose tail
@@ -373,19 +372,12 @@ __global__ void k_field_distance(fl_center_distance* centres, uint64_t ncentres,
   const double half = corner ? 0.0 : 0.5;
   const double L[3] = {c.x + half, c.y + half, c.z + half};
   const double w[3] = {ox + L[0] * h, oy + L[1] * h, oz + L[2] * h};
-  const double h2 = h * h;
   double best = __builtin_inf(), least = __builtin_inf();
   int32_t blo[3], bhi[3];
   for (int a = 0; a < 3; ++a) {
     blo[a] = 4 * G.bins.lo[a];
     bhi[a] = 4 * (G.bins.lo[a] + G.bins.dim[a]) - 1;
   }
-  // Lattice gap between the sample and sub-cell u on one axis (u covers [u + 1.5, u + 2.5)), less a
-  // slack for particles whose computed sub-cell rounding moved across a face.
-  auto gap = [&](int a, int32_t u) {
-    const double g = fmax(fmax((u + 1.5) - L[a], L[a] - (u + 2.5)), 0.0);
-    return fmax(g - 1e-6, 0.0);
-  };
   auto visit = [&](int32_t ux, int32_t uy, int32_t uz) {
     const int32_t b[3] = {static_cast<int32_t>(floor_div4(ux)), static_cast<int32_t>(floor_div4(uy)),
                           static_cast<int32_t>(floor_div4(uz))};
@@ -406,51 +398,7 @@ __global__ void k_field_distance(fl_center_distance* centres, uint64_t ncentres,
       }
     }
   };
-  int32_t plo[3] = {0, 0, 0}, phi[3] = {-1, -1, -1};  // the previous ring's cube (empty at first)
-  for (double rho = 1;;) {
-    int32_t lo[3], hi[3];
-    bool all = true;
-    for (int a = 0; a < 3; ++a) {
-      const double l = floor(L[a] - rho - 1.5), u = floor(L[a] + rho - 1.5);
-      lo[a] = l <= blo[a] ? blo[a] : static_cast<int32_t>(fmin(l, double(bhi[a]) + 1));
-      hi[a] = u >= bhi[a] ? bhi[a] : static_cast<int32_t>(fmax(u, double(blo[a]) - 1));
-      all = all && l <= blo[a] && u >= bhi[a];
-    }
-    // Sub-cells touching the sample first (they hold the nearest particle of a liquid sample, and lie in the
-    // first ring), then the rest of the ring; a plane, row or sub-cell whose box is farther than the least
-    // distance so far is skipped, and so is the run of a row that the previous ring visited.
-    for (int pass = rho == 1 ? 0 : 1; pass < 2; ++pass)
-      for (int32_t uz = lo[2]; uz <= hi[2]; ++uz) {
-        const double gz = gap(2, uz), gz2 = gz * gz;
-        if (pass == 0 ? gz != 0 : gz2 * h2 > best * (1 + 1e-9)) continue;
-        for (int32_t uy = lo[1]; uy <= hi[1]; ++uy) {
-          const double gy = gap(1, uy), gyz = gy * gy + gz2;
-          if (pass == 0 ? gy != 0 : gyz * h2 > best * (1 + 1e-9)) continue;
-          const bool inner = uy >= plo[1] && uy <= phi[1] && uz >= plo[2] && uz <= phi[2];
-          for (int32_t ux = lo[0]; ux <= hi[0]; ++ux) {
-            if (inner && ux == plo[0]) {
-              ux = phi[0];
-              continue;
-            }
-            const double gx = gap(0, ux);
-            const double g2 = gx * gx + gyz;
-            if ((g2 == 0) != (pass == 0)) continue;
-            if (g2 * h2 > best * (1 + 1e-9)) continue;
-            visit(ux, uy, uz);
-          }
-        }
-      }
-    for (int a = 0; a < 3; ++a) {
-      plo[a] = lo[a];
-      phi[a] = hi[a];
-    }
-    // Every unvisited particle lies at least (rho - rounding) cells from the sample.
-    const double reach = sqrt(best) * (1 + 1e-12);
-    if (finite(best) && reach < (rho - 1e-6) * h) break;
-    if (all) break;
-    // The next ring: twice as far, or just beyond the least distance once there is one.
-    rho = finite(best) ? fmin(2 * rho, reach / h * (1 + 1e-9) + 1e-5) : 2 * rho;
-  }
+  ring_walk(L, blo, bhi, h, best, visit);
   const double d = least - r;
   if (!finite(d)) {
     atomicMin(reinterpret_cast<unsigned long long*>(err), static_cast<unsigned long long>(error_word(i, kOutOfRange)));

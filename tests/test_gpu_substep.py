@@ -136,6 +136,23 @@ def test_device_built_components(ctx, n, share):
     assert np.array_equal(u.view(np.uint64), host["velocities"].view(np.uint64))
 
 
+@pytest.mark.parametrize("radius", [0.9, 1.3, 2.5, 5.0])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_field_of_detached_liquid(ctx, axis, radius):
+    """One particle and small clouds that begin 1.4 to 2.6 cells above a bin's first lattice coordinate (and on
+    either side of zero) along one axis: centre samples lie up to radius + 1 cells below the lowest bin."""
+    geom = O.geometry((0.0, 0.0, 0.0), 1.0)
+    rng = np.random.default_rng(axis)
+    for base in (0.0, -8.0):
+        for first in (1.4, 1.5, 1.6, 1.75, 1.89, 2.3, 2.6):
+            one = np.array([[3.0, 3.0, 3.0]])
+            cloud = 3.0 + np.vstack([np.zeros((1, 3)), rng.random((12, 3)) * 2.5])
+            for pos in (one, cloud):
+                pos = pos.copy()
+                pos[:, axis] += base + first - 3.0
+                check_field(ctx, geom, pos, radius)
+
+
 def test_substep_chain_matches_oracle(ctx):
     sc = scenes.dam_break(16, seed=3)
     geom = O.geometry((0.0, 0.0, 0.0), sc.h)
@@ -174,6 +191,33 @@ def test_substep_chain_matches_oracle(ctx):
         assert dv <= 1e-7 * speed
         assert dj <= 1e-10
         assert np.all(f == 1)
+
+
+@pytest.mark.parametrize("first", [1.6, 1.85, 3.3])
+def test_substep_of_a_detached_drop(ctx, first):
+    """One substep of a falling block of liquid, 5 x 4 x 5 cells, that touches no wall and begins at x = first
+    cells, against the oracle's chain (the bars of the chain test)."""
+    sc = scenes.dam_break(16, seed=6)
+    geom = O.geometry((0.0, 0.0, 0.0), sc.h)
+    h, radius, dt = sc.h, 0.9 * sc.h, 0.1 * sc.h
+    x0 = sc.positions[np.all(sc.positions < np.array([5, 4, 5]) * h, axis=1)]
+    x0 = x0 + np.array([first * h - x0[:, 0].min(), 6.2 * h, 5.4 * h])
+    v0 = np.array([0.3, -0.5, 0.1]) - 0.8 * (x0 - x0.mean(axis=0))  # falls and contracts
+    c0 = np.zeros((len(x0), 3, 3))
+    obstacle = SC.tank_obstacle()
+    assert ctx.scene_upload(geom, x0, v0, c0.reshape(-1, 9), sc.mass) == H.OK
+    o = H.substep_options(dt, field_radius=radius, capacity=1 << 16, obstacle=SC.obstacle_record(obstacle, R.OBSTACLE),
+                          pressure=H.pressure_options(relative_target=1e-10, levels=3, sweeps=2))
+    s, rep = ctx.substep(o)
+    assert s == H.OK, (s, int(rep["stage"]))
+    st, info = SC.oracle_substep(geom, SC.State(x0, v0, c0, sc.mass), dt, radius, obstacle,
+                                 O.pressure_options(relative_target=1e-12, levels=3, fp32=False), capacity=1 << 16)
+    assert rep["candidates"] == len(info["candidates"]) and rep["centre_samples"] == len(info["centres"])
+    assert rep["frozen_cells"] == len(info["frozen_cells"]) and rep["frozen_faces"] == len(info["frozen_faces"])
+    s, x, v, c, j, f = ctx.substep_download(len(x0))
+    speed = float(np.abs(st.v).max())
+    assert s == H.OK and np.abs(x - st.x).max() <= 1e-9 * h and np.abs(v - st.v).max() <= 1e-7 * speed
+    assert np.abs(j - st.ratio).max() <= 1e-10
 
 
 def test_failed_substep_leaves_the_scene(ctx):
