@@ -1962,6 +1962,15 @@ int fl_set_transfer_precision(fl_ctx* ctx, int bits) {
   return FL_OK;
 }
 
+// For the tests alone, and in no header: red-black V-cycles and PCG steps of this context with every half sweep
+// and step a launch of its own, against which the tiles, the single-workgroup levels and the single-launch
+// iterations are compared bit for bit.
+int fl_check_separate_launches(fl_ctx* ctx, int on) {
+  if (!ctx) return FL_FAILED_PRECONDITION;
+  ctx->separate_launches = on != 0;
+  return FL_OK;
+}
+
 int fl_substep(fl_ctx* ctx, const fl_substep_options* options, fl_substep_report* report) {
   if (!ctx || ctx->poisoned || !ctx->scene_loaded) return FL_FAILED_PRECONDITION;
   if (!options || !report) return FL_INVALID_ARGUMENT;

@@ -172,6 +172,7 @@ struct fl_ctx {
   void* substep = nullptr;    // SubstepBuffers (substep.hip)
   void* coupled = nullptr;    // CoupledBuffers (coupled.hip)
   void* uniform = nullptr;    // UniformBuffers (uniform.hip)
+  bool separate_launches = false;  // every half sweep and PCG step a launch of its own (fl_check_separate_launches)
 };
 
 namespace fl {

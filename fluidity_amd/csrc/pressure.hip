@@ -960,13 +960,15 @@ __global__ void k_restrict_all(const float* r, LevelViewT<KT> C) {
 // tiles) takes 1.88 ms instead of 2.52, one of 5712 (714 tiles; three sweeps) 6.27 instead of 6.78, one of 8320
 // (1120 tiles) 5.84 instead of 5.60, so the half sweeps stay apart from about three tiles per CU on.
 constexpr int kTileLanes = 512;
+constexpr int kTileReach = 4;                    // half sweeps of a launch at most, and blocks on a path to a halo cell
 constexpr uint64_t kTileLimit = 768;             // tiles of a level
 constexpr uint64_t kTileTable = 2 * kTileLimit;  // tiles of all levels of a hierarchy
 
 // Tile tables, one wave per coarse block: the level's blocks in the 4^3 around the tile's eight ((z,y,x)
-// order, -1 where there is none or none that a path of face neighbours from the tile leads to), then their
-// coarser blocks. Blocks without a coarse parent (no unknowns) belong to no tile: their values are zeroed here,
-// in both buffers.
+// order, -1 where there is none or none that a path of face neighbours from the tile leads to in as many steps
+// as a launch has half sweeps: a cell that many cells away may be reached through that many blocks, round missing
+// ones; with three steps its term was lost), then their coarser blocks. Blocks without a coarse parent (no
+// unknowns) belong to no tile: their values are zeroed here, in both buffers.
 __global__ __launch_bounds__(256) void k_tile_table(const int32_t* nbr, const int32_t* parent, uint64_t nb,
                                                     const int32_t* child, uint64_t tiles, int32_t* table, float* x,
                                                     float* r) {
@@ -981,7 +983,7 @@ __global__ __launch_bounds__(256) void k_tile_table(const int32_t* nbr, const in
   const bool inner = (bx == 1 || bx == 2) && (by == 1 || by == 2) && (bz == 1 || bz == 2);
   int id = -1;
   if (inner && c < tiles) id = child[8 * c + ((bz - 1) * 2 + (by - 1)) * 2 + (bx - 1)];
-  for (int round = 0; round < 3; ++round) {
+  for (int round = 0; round < kTileReach; ++round) {
     ids[w][t] = id;
     __syncthreads();
     if (id < 0) {
@@ -2132,8 +2134,9 @@ int build_levels(fl_ctx* ctx, Pressure& P, const std::vector<Key3>& blocks0, int
 
 // The first level of the single-workgroup cycle: at most kTailBlocks blocks there, kTailStore in all, and
 // kMaxTail levels. The number of levels if there is none (a large coarsest level).
-size_t tail_start(const Pressure& P) {
+size_t tail_start(const fl_ctx* ctx, const Pressure& P) {
   size_t l = P.levels.size();
+  if (ctx->separate_launches) return l;
   uint64_t blocks = 0;
   while (l > 0 && P.levels[l - 1].nb <= kTailBlocks && blocks + P.levels[l - 1].nb <= uint64_t(kTailStore) &&
          P.levels.size() - l < size_t(kMaxTail))
@@ -2168,7 +2171,7 @@ int setup_coefficients(fl_ctx* ctx, Pressure& P, const double* conductance = nul
     Level& F = P.levels[l];
     const Level& C = P.levels[l + 1];
     F.tiles = nullptr;
-    if (l >= tail_start(P) || C.nb > kTileLimit || used + C.nb > P.cap_tiles) continue;
+    if (l >= tail_start(ctx, P) || C.nb > kTileLimit || used + C.nb > P.cap_tiles) continue;
     int32_t* table = P.tile_table + 128 * used;
     used += C.nb;
     k_tile_table<<<static_cast<unsigned>((std::max(F.nb, C.nb) + 3) / 4), 256, 0, s>>>(F.nbr, F.parent, F.nb, C.child,
@@ -2247,7 +2250,7 @@ template <class KT>
 int vcycle(fl_ctx* ctx, Pressure& P, size_t l, int nu, int coarse_sweeps, int smoother) {
   hipStream_t s = ctx->stream;
   const size_t last = P.levels.size() - 1;
-  const size_t tail = tail_start(P);
+  const size_t tail = tail_start(ctx, P);
   if (l == last && l < tail) {  // a large coarsest level: grid-wide sweeps from zero
     const LevelViewT<KT> B = view<KT>(P, l);
     for (int pass = 0; pass < 4 * coarse_sweeps; ++pass) {
@@ -2272,7 +2275,7 @@ int vcycle(fl_ctx* ctx, Pressure& P, size_t l, int nu, int coarse_sweeps, int sm
     std::swap(P.levels[l].x, P.levels[l].r);  // the post-smoothed values are the level's x from here on
     return FL_OK;
   }
-  if (P.levels[l].tiles) {
+  if (P.levels[l].tiles && !ctx->separate_launches) {
     const unsigned tiles = static_cast<unsigned>(P.levels[l + 1].nb);
     const int32_t* table = P.levels[l].tiles;
     Level& F = P.levels[l];
@@ -2427,7 +2430,7 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
   diag.learned_iterations = 0;
   // A small system without the network (nor training pairs to collect) runs up to the next restart in one
   // launch; the others one iteration at a time.
-  const bool small = tail_start(P) == 0 && !use_net && !(net && net->collect_every > 0);
+  const bool small = tail_start(ctx, P) == 0 && !use_net && !(net && net->collect_every > 0);
   auto iterate = [&](uint64_t it) -> int {
     if (use_net) {
       k_tile_gather<<<static_cast<unsigned>(P.ntiles), 512, 0, s>>>(P.r32, L0.diag, P.cell_class, P.tile_blocks,
@@ -2603,7 +2606,7 @@ int time_levels(fl_ctx* ctx, Pressure& P, int reps, fl_kernel_time* out, size_t 
     put(FL_KERNEL_RESTRICT_RED, 0, n0, ms);
     FL_TRY(mean_ms(ctx, reps, [&] { k_prolong<KT><<<grid_for(n0), kThreads, 0, s>>>(V0, P.levels[1].x); }, &ms));
     put(FL_KERNEL_PROLONG, 0, n0, ms);
-    if (tail_start(P) > 1 && P.levels.size() > 2) {
+    if (tail_start(ctx, P) > 1 && P.levels.size() > 2) {
       const LevelViewT<KT> V2 = view<KT>(P, 2);
       const unsigned gb = static_cast<unsigned>((P.levels[1].nb + 3) / 4);
       FL_TRY(mean_ms(ctx, reps, [&] { k_block_smooth<KT, false><<<gb, 256, 0, s>>>(V1, nullptr, nullptr, nu); }, &ms));
@@ -2621,7 +2624,7 @@ int time_levels(fl_ctx* ctx, Pressure& P, int reps, fl_kernel_time* out, size_t 
     }
   }
   // The single-workgroup cycle of the small levels.
-  const size_t first = tail_start(P);
+  const size_t first = tail_start(ctx, P);
   if (first < P.levels.size()) {
     FL_TRY(mean_ms(ctx, reps, [&] { (void)run_tail<KT>(ctx, P, first, nu, P.last_coarse_sweeps); }, &ms));
     put(FL_KERNEL_TAIL_VCYCLE, static_cast<uint32_t>(first), P.levels[first].nb * 64, ms);

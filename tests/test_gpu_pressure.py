@@ -164,6 +164,55 @@ def test_level_wide_sweeps_by_tiles(ctx, minimum, extents, sweeps, bf16):
     np.testing.assert_allclose(out["velocities"], 0.0, atol=5e-6)
 
 
+def blocky_liquid(name):
+    """Liquid cells in 4^3 blocks [z, y, x]: L-shaped chains of five blocks whose ends a tile's corner cell depends on
+    around missing neighbours, blocks at random with every eighth cell missing, or fewer of them (small levels)."""
+    rng = np.random.default_rng(len(name))
+    b = np.zeros((12, 12, 12), bool)
+    if name == "chains":
+        for z, y, x in np.ndindex(3, 3, 3):
+            for dx, dy, dz in ((2, 2, 2), (1, 2, 2), (1, 1, 2), (1, 1, 1), (2, 1, 1)):
+                b[4 * z + dz, 4 * y + dy, 4 * x + dx] = True
+    elif name.startswith("small"):
+        b[3:7, 3:7, 3:7] = rng.random((4, 4, 4)) < float(name[5:])
+        b[3, 3, 3] = True
+    else:
+        b = rng.random(b.shape) < float(name)
+    liquid = b.repeat(4, 0).repeat(4, 1).repeat(4, 2)
+    return liquid if name == "chains" else liquid & (rng.random(liquid.shape) < 0.875)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("sweeps", [1, 2, 3, 5])
+@pytest.mark.parametrize("liquid", ["chains", "0.35", "0.55", "0.9", "small0.1", "small0.5", "small1"])
+def test_levels_in_one_launch_are_the_sweeps_one_by_one(ctx, liquid, sweeps, bf16):
+    """Tiles of up to four half sweeps, the small levels in one workgroup and (small systems) whole iterations in one
+    launch give the bits of the same solve with every half sweep and step a launch of its own, on liquids with
+    missing blocks and cells."""
+    cells = blocky_liquid(liquid)
+    n = len(cells)
+    sc = scenes.Scene("blocks", n, 0, cells, np.zeros((0, 3)), np.zeros((0, 3)), np.zeros((0, 3, 3)), 1.0)
+    b = np.arange(-1, n // 4 + 1)
+    z, y, x = np.meshgrid(b, b, b, indexing="ij")
+    blocks = np.zeros(x.size, R.INT3)
+    blocks["x"], blocks["y"], blocks["z"] = x.ravel(), y.ravel(), z.ravel()
+    faces = sc.pressure_faces(blocks, np.random.default_rng(1).normal(0.0, 1.0, 192 * len(blocks)))
+    args = (O.geometry((0.0, 0.0, 0.0), sc.h), blocks, 1e-3, sc.pressure_cells(), faces,
+            H.pressure_options(relative_target=1e-9, levels=4, sweeps=sweeps, bf16_levels=bf16))
+    s, got = ctx.project(*args)
+    assert H.lib().fl_check_separate_launches(ctx.handle, 1) == H.OK
+    try:
+        s_want, want = ctx.project(*args)
+    finally:
+        H.lib().fl_check_separate_launches(ctx.handle, 0)
+    assert s == s_want == H.OK
+    d, w = got["diagnostics"], want["diagnostics"]
+    print("iterations", d["iteration_count"], "restarts", d["restarts"], "levels", d["multigrid_level_count"], flush=True)
+    assert d["iteration_count"] == w["iteration_count"] and d["restarts"] == w["restarts"]
+    for name in ("pressures", "velocities"):
+        assert np.array_equal(got[name].view(np.uint64), want[name].view(np.uint64)), name
+
+
 @pytest.mark.parametrize("bf16,smoother", [(False, 1), (True, 1), (True, 2)], ids=["fp32_block", "bf16_block",
                                                                                "bf16_hybrid"])
 def test_block_smoother_meets_the_gates_deterministically(ctx, bf16, smoother):
