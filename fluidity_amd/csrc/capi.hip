@@ -688,6 +688,7 @@ int fl_reserve(fl_ctx* ctx) {
   // owned face slots.
   FL_TRY(grow_viscosity(ctx, nc, 6 * nc, nf));
   FL_TRY(grow_viscosity_terms(ctx, 18 * nc));
+  FL_TRY(fl::uniform_reserve(ctx));  // and the substep's velocity block of one viscosity
   FL_HIP(hipStreamSynchronize(ctx->stream));
   return FL_OK;
 }

@@ -427,6 +427,7 @@ struct UniformBlock {
 // the rows' structure, the Jacobi diagonal and the prescribed strains in base (link order); *rows counts the
 // strain rows that AssembleFullCellMacStrain3D would form. Failures also go to err (two words).
 int uniform_prepare(fl_ctx* ctx, UniformBlock* out);
+int uniform_reserve(fl_ctx* ctx);  // the same arrays, for the context's capacity of blocks
 int uniform_rows(fl_ctx* ctx, const CoupledSystem& S, const fl_pressure_cell* cells, double mu, double h, double dt,
                  double* base, uint64_t* err, uint64_t* rows);
 // As pcg_viscous_block, for the right-hand side in the block's rhs.

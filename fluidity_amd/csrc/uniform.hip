@@ -70,12 +70,7 @@ int take(T** p, uint64_t n) {
   return FL_OK;
 }
 
-int ensure(fl_ctx* ctx, uint64_t nb, UniformBuffers** out) {
-  if (!ctx->uniform) ctx->uniform = new (std::nothrow) UniformBuffers();
-  auto* B = static_cast<UniformBuffers*>(ctx->uniform);
-  if (!B) return FL_RESOURCE_EXHAUSTED;
-  *out = B;
-  if (nb <= B->cap_blocks && B->inertia) return FL_OK;
+int allocate(UniformBuffers* B, uint64_t nb) {
   B->release();
   const uint64_t n = nb * kBlockFaces;
   double** fv[] = {&B->inertia, &B->rhs, &B->v, &B->r, &B->z, &B->d[0], &B->d[1], &B->q, &B->diag, &B->uwall};
@@ -93,6 +88,22 @@ int ensure(fl_ctx* ctx, uint64_t nb, UniformBuffers** out) {
   }
   B->cap_blocks = nb;
   return FL_OK;
+}
+
+// Room for nb blocks: what is there, or what fl_reserve took for the context's capacity; else a quarter more
+// than asked for (within the capacity), so that a spreading liquid does not free and allocate in every substep.
+int ensure(fl_ctx* ctx, uint64_t nb, UniformBuffers** out) {
+  if (!ctx->uniform) ctx->uniform = new (std::nothrow) UniformBuffers();
+  auto* B = static_cast<UniformBuffers*>(ctx->uniform);
+  if (!B) return FL_RESOURCE_EXHAUSTED;
+  *out = B;
+  if (nb <= B->cap_blocks && B->host) return FL_OK;
+  const uint64_t more = std::min(nb + nb / 4, ctx->cap.blocks);
+  if (more > nb) {
+    if (allocate(B, more) == FL_OK) return FL_OK;
+    (void)hipGetLastError();  // the smaller try stands by itself
+  }
+  return allocate(B, nb);
 }
 
 // Weighted coefficient sqrt(dt) sqrt(w) c and strain weight mu h^3 2^k by exponent-separated products, as
@@ -508,6 +519,11 @@ __global__ void k_uniform_zero(uint64_t n, double* v, uint32_t* arrived) {
 }
 
 }  // namespace
+
+int uniform_reserve(fl_ctx* ctx) {
+  UniformBuffers* B = nullptr;
+  return ensure(ctx, std::max<uint64_t>(ctx->cap.blocks, 1), &B);
+}
 
 int uniform_prepare(fl_ctx* ctx, UniformBlock* out) {
   UniformBuffers* B = nullptr;

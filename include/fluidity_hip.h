@@ -444,9 +444,11 @@ int fl_device_name(fl_ctx* ctx, char* out, size_t size);
  * Create; attempt operations allocate and free nothing). fl_create itself reserves the projection's
  * arrays and its multigrid level pool from the pressure capacities. fl_reserve also reserves, from the
  * capacities, the device buffers that topology preparation, the boundary gather, the frozen geometry,
- * the pressure links and the particle update would otherwise allocate on first use: after it, every
- * call whose inputs stay within the capacities (at most 27 centre and 8 corner samples per candidate
- * cell, link fields at most one per cell or pressure face) allocates and frees no device memory. */
+ * the pressure links, the particle update and the viscous velocity blocks would otherwise allocate on
+ * first use: after it, every call whose inputs stay within the capacities (at most 27 centre and 8 corner
+ * samples per candidate cell, link fields at most one per cell or pressure face) allocates and frees no
+ * device memory, but for the sample, freeze and link arrays of fl_substep and the directions of the coupled
+ * viscous solve, which grow with the largest liquid they have met. */
 int fl_reserve(fl_ctx* ctx);
 
 /* ---- variational MAC viscosity (native/src/viscosity.cc; host/viscosity.h:47-160) ---- */

@@ -344,3 +344,45 @@ def test_uniform_viscosity_on_odd_grids(ctx, n):
     s, x, vel, c, j, f = ctx.substep_download(len(st.x))
     speed = max(float(np.abs(st.v).max()), 1e-3)
     assert s == H.OK and np.abs(x - st.x).max() <= 1e-9 * h and np.abs(vel - st.v).max() <= 1e-7 * speed
+
+
+def test_reserved_viscous_substep_of_more_blocks_allocates_nothing():
+    """After fl_reserve the velocity block of one viscosity lies in memory taken for the capacity: a liquid of few
+    cells in many more blocks than the one before it (every other array has held as much) allocates nothing."""
+    import ctypes as C
+
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    h = 1.0 / 32
+    rng = np.random.default_rng(3)
+    z, y, x = np.meshgrid(*[np.arange(24)] * 3, indexing="ij")
+    block = (np.stack([x, y, z], -1).reshape(-1, 3) + 0.5 + 0.2 * rng.random((24 ** 3, 3))) * (h / 2) + 8 * h
+    z, y, x = np.meshgrid(*[np.arange(4)] * 3, indexing="ij")
+    drops = (np.stack([x, y, z], -1).reshape(-1, 3) * 8 + 3.2 + rng.random((64, 3))) * h
+    floor = floor_record()
+    with H.Context(particles=1 << 16, blocks=1 << 12, lookup_blocks=1 << 16, pressure_cells=1 << 15,
+                   pressure_faces=1 << 17) as c:
+        assert H.lib().fl_reserve(c.handle) == H.OK
+
+        def step(pos, viscosity):
+            v = rng.normal(0.0, 0.1, pos.shape)
+            assert c.scene_upload(O.geometry((0.0, 0.0, 0.0), h), pos, v, np.zeros((len(pos), 9)), 1000.0 * h ** 3) == H.OK
+            o = H.substep_options(0.1 * h, field_radius=0.9 * h, capacity=1 << 16, obstacle=floor,
+                                  pressure=H.pressure_options(levels=2), dynamic_viscosity=viscosity)
+            s, rep = c.substep(o)
+            assert s == H.OK, (s, int(rep["stage"]))
+            return int(rep["blocks"]), int(rep["frozen_cells"]), int(rep["frozen_faces"])
+
+        step(block, 0.0)
+        many, few_cells, few_faces = step(drops, 0.0)
+        blocks, cells, faces = step(block, 1.0)
+        print("blocks", blocks, many, "cells", cells, few_cells, "faces", faces, few_faces, flush=True)
+        assert many > blocks + 256 and few_cells < cells and few_faces < faces
+        free = free_bytes()
+        step(drops, 1.0)
+        assert free_bytes() == free
