@@ -50,7 +50,7 @@ def g2p_algorithmic_bytes(n_particles, n_faces):
 
 # Algorithmic bytes per cell slot (64 per 4^3 block) of the projection kernels, each array counted once
 # per launch; cb is the byte width of a V-cycle coefficient (2 for BF16 storage, 4 for FP32). None: the
-# single-workgroup tail cycle over the smallest levels is latency-bound and not priced.
+# single workgroup's cycle and iteration over the smallest levels are latency-bound and not priced.
 def projection_bytes_per_slot(name, cb):
     return {
         # other colour's x, own b and diagonal, the three coefficient arrays, own x written
@@ -79,6 +79,13 @@ def projection_bytes_per_slot(name, cb):
         # per cell: p and seven FP64 cell arrays, six face ordinals, three 64-byte face records (each
         # face is shared by two cells), residual and defect written
         "k_evaluate": 8 + 56 + 24 + 192 + 16,
+        # b, diagonal and coefficients read, x written (level 0 by tiles)
+        "k_tile_smooth_pre": 12 + 3 * cb,
+        # every x, three coefficient arrays, red anchor, b and diagonal, coarse right-hand side (1/8) written
+        "k_residual_restrict": 10.5 + 3 * cb,
+        # x, b, diagonal, coefficients and coarse x (1/8) read, second buffer written
+        "k_tile_smooth_post": 16.5 + 3 * cb,
+        "k_small_pcg": None,
     }[name]
 
 

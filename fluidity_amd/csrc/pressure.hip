@@ -140,7 +140,8 @@ struct Pressure {
   int32_t* tile_table = nullptr;  // [cap_tiles][128]: Level::tiles
   uint64_t cap_tiles = 0;
   int levels_requested = 0;
-  int last_storage = 1, last_nu = 2, last_coarse_sweeps = 2;  // V-cycle settings of the last solve
+  int last_storage = 1, last_nu = 2, last_coarse_sweeps = 2, last_smoother = 0;  // V-cycle settings of the last solve
+  bool last_small = false;  // whether it ran whole iterations in one launch
   bool p_init_zero = false;  // warm start is identically zero: its evaluation equals the p = 0 one
   bool has_jump = false;
   // Frozen link coefficients and hierarchy coefficients of the current system for step duration
@@ -2390,6 +2391,7 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
   P.last_storage = opt.level_storage;
   P.last_nu = opt.smoothing_sweeps;
   P.last_coarse_sweeps = opt.coarse_sweeps;
+  P.last_smoother = opt.smoother;
   diag.restarts = 0;
   EvalResult e{};
   k_copy_f64<<<grid_for(P.nc), kThreads, 0, s>>>(P.nc, P.p_base, P.p);
@@ -2431,6 +2433,7 @@ int solve(fl_ctx* ctx, Pressure& P, const fl_pressure_options& opt, const Gates&
   // A small system without the network (nor training pairs to collect) runs up to the next restart in one
   // launch; the others one iteration at a time.
   const bool small = tail_start(ctx, P) == 0 && !use_net && !(net && net->collect_every > 0);
+  P.last_small = small;
   auto iterate = [&](uint64_t it) -> int {
     if (use_net) {
       k_tile_gather<<<static_cast<unsigned>(P.ntiles), 512, 0, s>>>(P.r32, L0.diag, P.cell_class, P.tile_blocks,
@@ -2595,18 +2598,45 @@ int time_levels(fl_ctx* ctx, Pressure& P, int reps, fl_kernel_time* out, size_t 
   const uint64_t n0 = L0.nb * 64;
   const LevelViewT<KT> V0 = view<KT>(P, 0);
   const int nu = std::max(P.last_nu, 1);
-  // Level-0 V-cycle kernels.
-  FL_TRY(mean_ms(ctx, reps, [&] { k_smooth<KT><<<grid_for(n0 / 2), kThreads, 0, s>>>(V0, 0, 0); }, &ms));
-  put(FL_KERNEL_SMOOTH, 0, n0, ms);
-  FL_TRY(mean_ms(ctx, reps, [&] { k_residual_red<KT><<<grid_for(n0 / 2), kThreads, 0, s>>>(V0, L0.r); }, &ms));
-  put(FL_KERNEL_RESIDUAL_RED, 0, n0, ms);
+  // Level-0 V-cycle kernels: by tiles (the first launch from zero and the one with the coarse correction), by half
+  // sweeps, or none of its own where level 0 is one of the single workgroup's.
+  const size_t first = tail_start(ctx, P);
+  const bool tiled = L0.tiles && !ctx->separate_launches && P.last_smoother != 1;
+  if (tiled) {
+    const LevelViewT<KT> V1 = view<KT>(P, 1);
+    const unsigned tiles = static_cast<unsigned>(P.levels[1].nb);
+    FL_TRY(mean_ms(ctx, reps, [&] {
+      if (nu >= 2)
+        k_tile_smooth<KT, 2, true, false, false><<<tiles, kTileLanes, 0, s>>>(V0, L0.tiles, L0.x, nullptr);
+      else
+        k_tile_smooth<KT, 1, true, false, false><<<tiles, kTileLanes, 0, s>>>(V0, L0.tiles, L0.x, nullptr);
+    }, &ms));
+    put(FL_KERNEL_TILE_SMOOTH_PRE, 0, n0, ms);
+    FL_TRY(mean_ms(ctx, reps, [&] { k_residual_restrict<KT><<<tiles, 256, 0, s>>>(V0, V1); }, &ms));
+    put(FL_KERNEL_RESIDUAL_RESTRICT, 0, n0, ms);
+    FL_TRY(mean_ms(ctx, reps, [&] {
+      const float* xc = P.levels[1].x;
+      if (nu >= 2)
+        k_tile_smooth<KT, 2, false, true, true><<<tiles, kTileLanes, 0, s>>>(V0, L0.tiles, L0.r, xc);
+      else
+        k_tile_smooth<KT, 1, false, true, true><<<tiles, kTileLanes, 0, s>>>(V0, L0.tiles, L0.r, xc);
+    }, &ms));
+    put(FL_KERNEL_TILE_SMOOTH_POST, 0, n0, ms);
+  } else if (first > 0) {
+    FL_TRY(mean_ms(ctx, reps, [&] { k_smooth<KT><<<grid_for(n0 / 2), kThreads, 0, s>>>(V0, 0, 0); }, &ms));
+    put(FL_KERNEL_SMOOTH, 0, n0, ms);
+    FL_TRY(mean_ms(ctx, reps, [&] { k_residual_red<KT><<<grid_for(n0 / 2), kThreads, 0, s>>>(V0, L0.r); }, &ms));
+    put(FL_KERNEL_RESIDUAL_RED, 0, n0, ms);
+  }
   if (P.levels.size() > 1) {
     const LevelViewT<KT> V1 = view<KT>(P, 1);
-    FL_TRY(mean_ms(ctx, reps, [&] { k_restrict_red<KT><<<grid_for(V1.n), kThreads, 0, s>>>(L0.r, V1); }, &ms));
-    put(FL_KERNEL_RESTRICT_RED, 0, n0, ms);
-    FL_TRY(mean_ms(ctx, reps, [&] { k_prolong<KT><<<grid_for(n0), kThreads, 0, s>>>(V0, P.levels[1].x); }, &ms));
-    put(FL_KERNEL_PROLONG, 0, n0, ms);
-    if (tail_start(ctx, P) > 1 && P.levels.size() > 2) {
+    if (!tiled && first > 0) {
+      FL_TRY(mean_ms(ctx, reps, [&] { k_restrict_red<KT><<<grid_for(V1.n), kThreads, 0, s>>>(L0.r, V1); }, &ms));
+      put(FL_KERNEL_RESTRICT_RED, 0, n0, ms);
+      FL_TRY(mean_ms(ctx, reps, [&] { k_prolong<KT><<<grid_for(n0), kThreads, 0, s>>>(V0, P.levels[1].x); }, &ms));
+      put(FL_KERNEL_PROLONG, 0, n0, ms);
+    }
+    if (first > 1 && P.levels.size() > 2) {
       const LevelViewT<KT> V2 = view<KT>(P, 2);
       const unsigned gb = static_cast<unsigned>((P.levels[1].nb + 3) / 4);
       FL_TRY(mean_ms(ctx, reps, [&] { k_block_smooth<KT, false><<<gb, 256, 0, s>>>(V1, nullptr, nullptr, nu); }, &ms));
@@ -2624,25 +2654,31 @@ int time_levels(fl_ctx* ctx, Pressure& P, int reps, fl_kernel_time* out, size_t 
     }
   }
   // The single-workgroup cycle of the small levels.
-  const size_t first = tail_start(ctx, P);
   if (first < P.levels.size()) {
     FL_TRY(mean_ms(ctx, reps, [&] { (void)run_tail<KT>(ctx, P, first, nu, P.last_coarse_sweeps); }, &ms));
     put(FL_KERNEL_TAIL_VCYCLE, static_cast<uint32_t>(first), P.levels[first].nb * 64, ms);
   }
-  // PCG kernels on level 0 (FP32 vectors and coefficients).
-  const unsigned rg = reduce_grid(n0);
-  FL_TRY(mean_ms(ctx, reps, [&] {
-    k_direction_apply<<<rg, kThreads, 0, s>>>(n0, L0.nbr, L0.k, L0.anchor, L0.diag, L0.x, P.d32, P.dn32, P.q32,
-                                              P.fscal, 0, P.partial);
-  }, &ms));
-  put(FL_KERNEL_DIRECTION_APPLY, 0, n0, ms);
-  FL_TRY(mean_ms(ctx, reps, [&] {
-    k_update_xr<<<rg, kThreads, 0, s>>>(n0, P.d32, P.q32, L0.diag, P.fine_vol, P.x32, P.r32, P.fscal, P.partial,
-                                        P.perr);
-  }, &ms));
-  put(FL_KERNEL_UPDATE_XR, 0, n0, ms);
-  FL_TRY(mean_ms(ctx, reps, [&] { k_dot<<<rg, kThreads, 0, s>>>(n0, P.r32, L0.x, P.partial); }, &ms));
-  put(FL_KERNEL_DOT, 0, n0, ms);
+  // PCG kernels on level 0 (FP32 vectors and coefficients), or the iteration in one launch (the residual is left as
+  // it is, so that every repetition is the same one).
+  if (first == 0 && P.last_small) {
+    const SmallPcg A{L0.k, L0.diag, P.fine_vol, P.x32, P.dn32, P.d32, P.q32, P.scal, P.fscal, P.perr, 1, 0.0, 0.0, -1.0};
+    FL_TRY(mean_ms(ctx, reps, [&] { (void)run_small_pcg<KT>(ctx, P, nu, P.last_coarse_sweeps, A); }, &ms));
+    put(FL_KERNEL_SMALL_PCG, 0, n0, ms);
+  } else {
+    const unsigned rg = reduce_grid(n0);
+    FL_TRY(mean_ms(ctx, reps, [&] {
+      k_direction_apply<<<rg, kThreads, 0, s>>>(n0, L0.nbr, L0.k, L0.anchor, L0.diag, L0.x, P.d32, P.dn32, P.q32,
+                                                P.fscal, 0, P.partial);
+    }, &ms));
+    put(FL_KERNEL_DIRECTION_APPLY, 0, n0, ms);
+    FL_TRY(mean_ms(ctx, reps, [&] {
+      k_update_xr<<<rg, kThreads, 0, s>>>(n0, P.d32, P.q32, L0.diag, P.fine_vol, P.x32, P.r32, P.fscal, P.partial,
+                                          P.perr);
+    }, &ms));
+    put(FL_KERNEL_UPDATE_XR, 0, n0, ms);
+    FL_TRY(mean_ms(ctx, reps, [&] { k_dot<<<rg, kThreads, 0, s>>>(n0, P.r32, L0.x, P.partial); }, &ms));
+    put(FL_KERNEL_DOT, 0, n0, ms);
+  }
   // The FP64 evaluation of the accepted pressure (recomputes the same residuals and defects).
   const unsigned g = reduce_grid(P.nc, kPartials);
   FL_TRY(mean_ms(ctx, reps, [&] {

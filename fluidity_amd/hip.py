@@ -157,7 +157,8 @@ class KernelTime(C.Structure):
 
 KERNEL_NAMES = ("k_smooth", "k_residual_red", "k_restrict_red", "k_prolong", "k_block_smooth_pre",
                 "k_block_smooth_post", "k_residual_all", "k_restrict_all", "k_tail_vcycle", "k_direction_apply",
-                "k_update_xr", "k_dot", "k_evaluate")
+                "k_update_xr", "k_dot", "k_evaluate", "k_tile_smooth_pre", "k_residual_restrict", "k_tile_smooth_post",
+                "k_small_pcg")
 
 
 class Context:

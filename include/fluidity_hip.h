@@ -839,7 +839,13 @@ enum {
   FL_KERNEL_DIRECTION_APPLY = 9,   /* d = z + beta d, q = A d, d . q (FP32, FP64 partials) */
   FL_KERNEL_UPDATE_XR = 10,        /* x += alpha d, r -= alpha q, residual norms */
   FL_KERNEL_DOT = 11,              /* r . z */
-  FL_KERNEL_EVALUATE = 12          /* FP64 residual, defect and identity check */
+  FL_KERNEL_EVALUATE = 12,         /* FP64 residual, defect and identity check */
+  /* where level 0 is smoothed by tiles, in place of the first four */
+  FL_KERNEL_TILE_SMOOTH_PRE = 13,  /* the first launch of the pre-smoothing, up to two sweeps from zero */
+  FL_KERNEL_RESIDUAL_RESTRICT = 14, /* residual of the red cells and its sums */
+  FL_KERNEL_TILE_SMOOTH_POST = 15, /* the first launch of the post-smoothing, coarse correction and up to two sweeps */
+  /* where level 0 is one of the single workgroup's, in place of the first four and 9 to 11 */
+  FL_KERNEL_SMALL_PCG = 16         /* one whole iteration */
 };
 typedef struct fl_kernel_time {
   uint32_t kernel;

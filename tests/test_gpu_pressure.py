@@ -213,6 +213,31 @@ def test_levels_in_one_launch_are_the_sweeps_one_by_one(ctx, liquid, sweeps, bf1
         assert np.array_equal(got[name].view(np.uint64), want[name].view(np.uint64)), name
 
 
+@pytest.mark.parametrize("extents,levels,smoother,ran", [
+    ((48, 48, 40), 4, 0, {"k_tile_smooth_pre", "k_residual_restrict", "k_tile_smooth_post", "k_update_xr"}),
+    ((48, 48, 40), 4, 1, {"k_smooth", "k_prolong", "k_update_xr"}),
+    ((48, 48, 40), 1, 0, {"k_smooth", "k_residual_red", "k_dot"}),
+    ((8, 8, 8), 2, 0, {"k_small_pcg", "k_tail_vcycle"})])
+def test_timed_kernels_are_those_that_run(ctx, extents, levels, smoother, ran):
+    """The per-kernel times name level 0's kernels by what the last projection launched there."""
+    geom, sb, cells, faces, _ = K.affine_problem(0, extents, True)
+    opt = H.pressure_options(relative_target=1e-6, levels=levels)
+    opt["smoother"] = smoother
+    s, first = ctx.project(geom, sb, 1.0, cells, faces, opt)
+    assert s == H.OK
+    s, rows = ctx.time_projection_kernels(3)
+    assert s == H.OK
+    level0 = {H.KERNEL_NAMES[k] for k, level, _, ms in rows if level == 0 and ms > 0.0}
+    choice = {"k_smooth", "k_residual_red", "k_restrict_red", "k_prolong", "k_tile_smooth_pre", "k_residual_restrict",
+              "k_tile_smooth_post", "k_small_pcg", "k_tail_vcycle", "k_direction_apply", "k_update_xr", "k_dot"}
+    print(sorted(level0), flush=True)
+    assert ran <= level0
+    assert not ("k_smooth" in level0 and "k_tile_smooth_pre" in level0)
+    assert ("k_small_pcg" in level0) != ("k_update_xr" in level0) and level0 <= choice | {"k_evaluate"}
+    s, again = ctx.project(geom, sb, 1.0, cells, faces, opt)
+    assert s == H.OK and np.array_equal(first["pressures"].view(np.uint64), again["pressures"].view(np.uint64))
+
+
 @pytest.mark.parametrize("bf16,smoother", [(False, 1), (True, 1), (True, 2)], ids=["fp32_block", "bf16_block",
                                                                                "bf16_hybrid"])
 def test_block_smoother_meets_the_gates_deterministically(ctx, bf16, smoother):
