@@ -45,12 +45,6 @@ uint64_t layer_offset(int l) {
   return o;
 }
 
-__device__ inline void tap(int k, int& dz, int& dy, int& dx) {
-  dz = k / 9 - 1;
-  dy = (k / 3) % 3 - 1;
-  dx = k % 3 - 1;
-}
-
 // ---- FP32 convolutions (training) ----
 // A 3x3x3 convolution of zero-padded cubes as a register tile: a lane holds VX voxels of one row and CO
 // output channels, reads VX + 2 values per input row from LDS and feeds 3 VX CO multiply-adds from them,
