@@ -64,13 +64,13 @@ int net_infer(hipStream_t s, const float* params, void* frags, float* act, uint6
 // Masked loss: scalars[0] = sum of the liquid mask, scalars[1] = loss; writes dL/dout into grad.
 int net_loss(hipStream_t s, const float* act, const float* target, float* grad, uint64_t nt, float* partial,
              float* scalars);
-// Backward pass of the last net_forward (its packed weights): grad must be zero except dL/dout at kActOut;
-// writes every parameter gradient and leaves dL/dinput at kActIn of each gradient record.
 // Tile chunks with partial parameter gradients of their own: two workgroups of the weights' gradients for each of
 // the 256 CUs (their LDS leaves room for two), more only add partials to reduce. Past it the chunks grow by whole
 // tiles, so 513 tiles make 257 chunks of two: loss and gradients of 512 / 513 / 600 / 1024 tiles take 1.86 / 2.13 /
 // 2.38 / 2.90 ms.
 constexpr uint64_t kGradChunks = 512;
+// Backward pass of the last net_forward (its packed weights): grad must be zero except dL/dout at kActOut;
+// writes every parameter gradient and leaves dL/dinput at kActIn of each gradient record.
 int net_backward(hipStream_t s, const float* packed, const float* act, float* grad, uint64_t nt, float* partial,
                  uint64_t partial_floats, float* grad_params);
 int net_clear(hipStream_t s, float* p, uint64_t n);
