@@ -398,7 +398,9 @@ typedef struct fl_pressure_options {
   int32_t smoother;                    /* 0 red-black Gauss-Seidel half sweeps over the whole level; 1 block
                                           smoother: red-black sweeps inside each 4^3 block with the block's
                                           neighbours held fixed (block Jacobi between blocks); 2 level-wide
-                                          sweeps on the finest level, the block smoother on coarser ones */
+                                          sweeps on the finest level, the block smoother on coarser ones. The
+                                          levels of at most 64 blocks (92 together) take level-wide sweeps
+                                          under each */
 } fl_pressure_options;
 
 typedef struct fl_pressure_diagnostics {
